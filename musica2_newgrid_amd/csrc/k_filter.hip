@@ -735,17 +735,12 @@ hipError_t launch_shock_wall(const FilterArgs &a, int axis, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Tiles of the filters: chunks of >= 16 planes, about 1024 workgroups per block.
-TileRange filter_tiles(const Geom &g, int kc_req) {
+// Tiles of the filters: 32x16, chunks of kc planes.
+TileRange filter_tiles(const Geom &g, int kc) {
   TileRange t{};
   t.tiles_x = (g.nx + FX - 1) / FX;
   t.tiles_y = (g.ny + FY - 1) / FY;
-  const long nxy = (long)t.tiles_x * t.tiles_y;
-  const long want = (1024 + nxy - 1) / nxy;
-  int kc = kc_req > 0 ? kc_req : (int)((g.nz + want - 1) / want);
-  if (kc_req <= 0 && kc < 16) kc = nxy * ((g.nz + 15) / 16) >= 512 ? 16 : (kc < 4 ? 4 : kc);
-  if (kc > g.nz) kc = g.nz;
-  t.kchunk = kc;
+  t.kchunk = kc < 1 ? 1 : (kc > g.nz ? g.nz : kc);
   return t;
 }
 

@@ -329,19 +329,13 @@ __global__ __launch_bounds__(TX *TY, 2) void k_visc(const Batch<ViscArgs> *__res
   }
 }
 
-// Tiles of the 32x16 viscous kernels: chunks of >= 16 planes, about 2048
-// workgroups per block (4 per CU slot of 256 CUs x 2).
+// Tiles of the viscous kernels: 32x16, chunks of kc planes.
 constexpr int VX = 32, VY = 16;
-TileRange vtiles(const Geom &g, int kc_req) {
+TileRange vtiles(const Geom &g, int kc) {
   TileRange t{};
   t.tiles_x = (g.nx + VX - 1) / VX;
   t.tiles_y = (g.ny + VY - 1) / VY;
-  const long nxy = (long)t.tiles_x * t.tiles_y;
-  const long want = (2048 + nxy - 1) / nxy;
-  int kc = kc_req > 0 ? kc_req : (int)((g.nz + want - 1) / want);
-  if (kc_req <= 0 && kc < 16) kc = nxy * ((g.nz + 15) / 16) >= 512 ? 16 : (kc < 4 ? 4 : kc);
-  if (kc > g.nz) kc = g.nz;
-  t.kchunk = kc;
+  t.kchunk = kc < 1 ? 1 : (kc > g.nz ? g.nz : kc);
   return t;
 }
 

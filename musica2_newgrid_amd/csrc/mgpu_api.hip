@@ -799,19 +799,83 @@ int setup_exchange(mgpu_handle *h) {
   return 0;
 }
 
-// Default k-chunk: aim at >= 2048 workgroups, at least 32 planes per chunk
-// (the 10-plane queue warm-up is paid once per chunk), but at least 8 planes
-// only on blocks too small to give every CU a workgroup otherwise.
-int kchunk_for(const Geom &g, int shape) {
-  const int TX = kStageShapes[shape][0], TY = kStageShapes[shape][1];
-  const long nxy = (long)((g.nx + TX - 1) / TX) * ((g.ny + TY - 1) / TY);
-  long want = (2048 + nxy - 1) / nxy;
-  if (want < 1) want = 1;
-  long kc = (g.nz + want - 1) / want;
-  const long kmin = nxy * ((g.nz + 31) / 32) >= 512 ? 32 : 8;
-  if (kc < kmin) kc = kmin;
-  if (kc > g.nz) kc = g.nz;
-  return (int)kc;
+// How many workgroups of a k-marching kernel the chip holds at once
+// (`slots`), and the time of one plane, in units of a 64x8 stage workgroup's:
+// `alone` while every workgroup has a CU for itself, `shared` beyond that.
+struct MarchCost {
+  int tx, ty, slots;
+  double alone, shared;
+};
+
+// Planes per workgroup of one batched launch that has not been tuned: the
+// workgroups run in ceil(workgroups / slots) rounds, and a round costs its
+// planes plus about two for the launch and the queue warm-up (64x8 tiles on
+// 512x256x128, 3-D curvilinear: 905 us in chunks of 128 planes, 926 / 951 /
+// 983 / 1100 us in chunks of 64 / 32 / 16 / 8, where rounds * (planes + 2)
+// says 919 / 947 / 1002 / 1114).  One number for all blocks of the batch, as
+// they share the rounds.  At 64^3 two planes instead of eight: the march is
+// then a chain of two plane latencies of about 3 us.
+int plan_kchunk(const mgpu_handle *h, const MarchCost &m, double *cost) {
+  int maxnz = 1;
+  for (const auto &bd : h->b) maxnz = bd.g.nz > maxnz ? bd.g.nz : maxnz;
+  double best = 1e30;
+  int best_kc = 1;
+  for (int kc = 1; kc <= maxnz; kc++) {
+    // chunk lengths that only unbalance the last chunk are skipped by the
+    // strict comparison below
+    long nt = 0;
+    for (const auto &bd : h->b)
+      nt += (long)((bd.g.nx + m.tx - 1) / m.tx) * ((bd.g.ny + m.ty - 1) / m.ty) * ((bd.g.nz + kc - 1) / kc);
+    const long rounds = (nt + m.slots - 1) / m.slots;
+    const double t = (double)rounds * (kc + 2) * (nt <= kCUs ? m.alone : m.shared);
+    if (t < best) {
+      best = t;
+      best_kc = kc;
+    }
+  }
+  if (cost) *cost = best;
+  return best_kc;
+}
+
+// Stage tiles: 512-thread workgroups fill a CU (139 / 120 KB of LDS), of the
+// 256-thread ones (67 / 73 KB) two share one.  A lone 16x16 or 32x8 plane
+// takes 2.75 us where a 64x8 one takes 3.4 (16^3 and 64^3, Cartesian), a
+// pair of them 1.04 to 1.07 of it at the same number of points (more halo
+// per point; 192^3, 161x97x65 c3).  64x4 was never the fastest.
+MarchCost stage_cost(int shape) {
+  const bool half = kStageShapes[shape][0] * kStageShapes[shape][1] == 256;
+  return {kStageShapes[shape][0], kStageShapes[shape][1], half ? 2 * kCUs : kCUs, half ? 0.8 : 1.0,
+          half ? 1.06 : (kStageShapes[shape][0] == 32 ? 1.03 : 1.0)};
+}
+
+// Tile shape and k-chunk of stage variant v: the tuned ones, else the
+// cheapest of the classic shapes by the rule above.
+void stage_plan(const mgpu_handle *h, int v, int &shape, int &kc) {
+  shape = h->shape[v];
+  kc = h->kchunk[v];
+  if (!h->shape_auto[v]) {
+    if (kc <= 0) kc = plan_kchunk(h, stage_cost(shape), nullptr);
+    return;
+  }
+  double best = 1e30;
+  for (int sh : {2, 4, 1, 3}) {
+    double t;
+    const int k = plan_kchunk(h, stage_cost(sh), &t);
+    if (t < best) {
+      best = t;
+      shape = sh;
+      kc = k;
+    }
+  }
+}
+
+// k-chunk of k_visc (kind 0), k_vdiv (1) and the filter (2), all 32x16 tiles
+// of 512 threads: one workgroup per CU at their register counts, but two of
+// k_vdiv on Cartesian and 2.5-D blocks (120 VGPRs).
+int aux_kchunk(const mgpu_handle *h, int kind) {
+  if (h->kc_aux[kind] > 0) return h->kc_aux[kind];
+  const bool two = kind == 1 && h->c.curvilinear != MGPU_GEOM_C3;
+  return plan_kchunk(h, MarchCost{32, 16, two ? 2 * kCUs : kCUs, 1.0, two ? 1.5 : 1.0}, nullptr);
 }
 
 // Process-wide cache of tuned stage parameters, keyed by block geometry and
@@ -919,10 +983,10 @@ StageArgs stage_args(const mgpu_handle *h, const BlockData &bd, int in, int s0, 
 // the launch's tile count.
 int stage_ranges(const mgpu_handle *h, int v, std::vector<TileRange> &tr) {
   tr.clear();
-  int first = 0;
+  int first = 0, shape, kc;
+  stage_plan(h, v, shape, kc);
   for (const auto &bd : h->b) {
-    const int kc = h->kchunk[v] > 0 ? h->kchunk[v] : kchunk_for(bd.g, h->shape[v]);
-    TileRange t = stage_tiles(bd.g, h->shape[v], kc);
+    TileRange t = stage_tiles(bd.g, shape, kc);
     t.jfirst = h->jfirst[v];
     t.first = first;
     first += tile_count(t, bd.g.nz);
@@ -1015,8 +1079,12 @@ int build_tables(mgpu_handle *h) {
     return 0;
   }
   std::vector<TileRange> tr[2];
-  h->nt_stage[0] = stage_ranges(h, 0, tr[0]);
-  h->nt_stage[1] = stage_ranges(h, 1, tr[1]);
+  for (int v = 0; v < 2; v++) {
+    int kc;
+    h->nt_stage[v] = stage_ranges(h, v, tr[v]);
+    stage_plan(h, v, h->run_shape[v], kc);
+  }
+  const int kcv = aux_kchunk(h, 0), kcd = aux_kchunk(h, 1), kcf = aux_kchunk(h, 2);
   std::vector<Batch<StageArgs>> st((size_t)3 * nrk * nb);
   std::vector<Batch<ViscArgs>> vi(3 * nb);
   std::vector<Batch<VdivArgs>> vd(nb);
@@ -1025,8 +1093,7 @@ int build_tables(mgpu_handle *h) {
   int fv = 0, fd = 0, ff = 0;
   for (int b = 0; b < nb; b++) {
     const BlockData &bd = h->b[b];
-    TileRange tv = visc_tiles(bd.g, h->kc_aux[0]), td = vdiv_tiles(bd.g, h->kc_aux[1]),
-              tf = filter_tiles(bd.g, h->kc_aux[2]);
+    TileRange tv = visc_tiles(bd.g, kcv), td = vdiv_tiles(bd.g, kcd), tf = filter_tiles(bd.g, kcf);
     tv.jfirst = h->jf_aux[0];
     td.jfirst = h->jf_aux[1];
     tf.jfirst = h->jf_aux[2];
@@ -1279,7 +1346,7 @@ int enqueue_step(mgpu_handle *h, int s0) {
       ProfScope ps(h, MGPU_K_STAGE);
       const int v = (last && visc) ? 1 : 0;
       HIPCK(h, launch_stage(h->d_stage + ((size_t)s0 * nrk + (irk - 1)) * nb, nb, h->nt_stage[v], geo,
-                            last && visc, h->shape[v], stage_mode(h, irk), stage_wall(h), h->stream));
+                            last && visc, h->run_shape[v], stage_mode(h, irk), stage_wall(h), h->stream));
     }
     if (h->mixed && !last) {
       ProfScope ps(h, MGPU_K_HALO);
@@ -1412,8 +1479,14 @@ int handle_new(const mgpu_case &c, mgpu_handle **out) {
   h->use_graph = (c.launch_flags & MGPU_LAUNCH_EAGER) == 0;
   h->stage_family = (c.launch_flags & MGPU_LAUNCH_STAGE_PIPELINED) ? 2
                     : ((c.launch_flags & MGPU_LAUNCH_STAGE_CLASSIC) ? 1 : 0);
-  if (h->stage_family == 2) h->shape[0] = h->shape[1] = kFirstPipelinedShape;
+  if (h->stage_family == 2) {
+    h->shape[0] = h->shape[1] = kFirstPipelinedShape;
+    h->shape_auto[0] = h->shape_auto[1] = false;
+  }
   h->mixed = c.precision == MGPU_PREC_MIXED;
+  // mixed precision keeps 64x8 until it is tuned: the compiler contracts the
+  // FP32 sums of the shapes differently (1e-8 of a step's increment)
+  if (h->mixed) h->shape_auto[0] = h->shape_auto[1] = false;
   if (hipGetDevice(&h->device) != hipSuccess) {
     delete h;
     return fail(nullptr, MGPU_EDEVICE, "no HIP device");
@@ -1956,7 +2029,7 @@ int tune_aux(mgpu_handle *h, bool force, hipEvent_t e0, hipEvent_t e1) {
         int first = 0;
         for (int b = 0; b < nb; b++) {
           tab[b].a = filter_args(h, h->b[b], s0, sa);
-          tab[b].t = filter_tiles(h->b[b].g, kc);
+          tab[b].t = filter_tiles(h->b[b].g, aux_kchunk(h, 2));
           tab[b].t.jfirst = jf;
           tab[b].t.first = first;
           first += tile_count(tab[b].t, h->b[b].g.nz);
@@ -2214,6 +2287,7 @@ int mgpu_autotune(mgpu_handle *h, int flags) {
       std::lock_guard<std::mutex> lk(g_tune_mu);
       auto it = g_tune_cache.find(key);
       if (it != g_tune_cache.end()) {
+        h->shape_auto[v] = false;
         h->shape[v] = it->second.first & 0xff;
         h->jfirst[v] = it->second.first >> 8;
         h->kchunk[v] = it->second.second;
@@ -2226,6 +2300,7 @@ int mgpu_autotune(mgpu_handle *h, int flags) {
     float best = 1e30f;
     int best_shape = h->shape[v], best_kc = h->kchunk[v], best_jf = h->jfirst[v];
     const int kcs[] = {0, 4, 8, 16, 32, 64, 128, 256};
+    h->shape_auto[v] = false;
     int maxnz = 0;
     for (const auto &bd : h->b) maxnz = bd.g.nz > maxnz ? bd.g.nz : maxnz;
     std::vector<Batch<StageArgs>> tab(nb);
@@ -2289,19 +2364,19 @@ int mgpu_stage_config(mgpu_handle *h, int block, int variant, int *shape_tx, int
   const BlockData &bd = h->b[block];
   if (variant >= 2) {
     const int kind = variant - 2;
-    const TileRange t = kind == 0 ? visc_tiles(bd.g, h->kc_aux[0])
-                                  : (kind == 1 ? vdiv_tiles(bd.g, h->kc_aux[1]) : filter_tiles(bd.g, h->kc_aux[2]));
+    const int kc = aux_kchunk(h, kind);
+    const TileRange t =
+        kind == 0 ? visc_tiles(bd.g, kc) : (kind == 1 ? vdiv_tiles(bd.g, kc) : filter_tiles(bd.g, kc));
     if (shape_tx) *shape_tx = 32;  // the viscous kernels and the filters use 32x16 tiles
     if (shape_ty) *shape_ty = 16;
     if (kchunk) *kchunk = t.kchunk;
     return 0;
   }
-  if (shape_tx) *shape_tx = kStageShapes[h->shape[variant]][0];
-  if (shape_ty) *shape_ty = kStageShapes[h->shape[variant]][1];
-  if (kchunk) {
-    const int kc = h->kchunk[variant] > 0 ? h->kchunk[variant] : kchunk_for(bd.g, h->shape[variant]);
-    *kchunk = stage_tiles(bd.g, h->shape[variant], kc).kchunk;
-  }
+  int shape, kc;
+  stage_plan(h, variant, shape, kc);
+  if (shape_tx) *shape_tx = kStageShapes[shape][0];
+  if (shape_ty) *shape_ty = kStageShapes[shape][1];
+  if (kchunk) *kchunk = stage_tiles(bd.g, shape, kc).kchunk;
   return 0;
 }
 

@@ -94,12 +94,15 @@ struct mgpu_handle {
   bool exchange_ready = false;
   bool ghosts_dirty = false;
   // stage kernel launch parameters: [0] Euler stages, [1] last stage with the
-  // viscous divergence (chosen by mgpu_autotune, else a default); kchunk 0
-  // means the per-block default
+  // viscous divergence, as mgpu_autotune chose them; shape_auto / kchunk 0:
+  // not tuned, chosen by size when the tables are built (run_shape: the
+  // shape the tables are built for)
   int shape[2] = {2, 2};
+  bool shape_auto[2] = {true, true};
+  int run_shape[2] = {2, 2};
   int stage_family = 0;  // 0: the tuner may pick either stage kernel, 1: classic only, 2: pipelined only
   int kchunk[2] = {0, 0};
-  // planes per workgroup of k_visc, k_vdiv and the filter (0: per-block default)
+  // planes per workgroup of k_visc, k_vdiv and the filter (0: chosen by size)
   int kc_aux[3] = {0, 0, 0};
   // tile numbering (TileRange::jfirst) of the stage variants and of k_visc,
   // k_vdiv and the filter

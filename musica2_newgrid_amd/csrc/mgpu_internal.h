@@ -121,6 +121,7 @@ __device__ __forceinline__ void stg_nt(float *b, idx_t i, float v) { __builtin_n
 // of logical tiles: neighbouring tiles (which re-read each other's halos)
 // then share an L2.  Bijective for any count n.
 constexpr int NXCD = 8;
+constexpr int kCUs = 256;
 __device__ __forceinline__ int xcd_remap(int w, int n) {
   const int x = w % NXCD, l = w / NXCD;
   const int q = n / NXCD, r = n % NXCD;
@@ -464,7 +465,7 @@ TileRange stage_tiles(const Geom &g, int shape, int kchunk);
 // wall rows (is_wall2; classic shapes only)
 hipError_t launch_stage(const Batch<StageArgs> *tab, int nb, int ntiles, int geo, bool visc, int shape,
                         int mode, int wall, hipStream_t s);
-TileRange visc_tiles(const Geom &g, int kchunk);  // kchunk 0: default
+TileRange visc_tiles(const Geom &g, int kchunk);
 hipError_t launch_visc(const Batch<ViscArgs> *tab, int nb, int ntiles, int geo, hipStream_t s);
 TileRange vdiv_tiles(const Geom &g, int kchunk);
 hipError_t launch_vdiv(const Batch<VdivArgs> *tab, int nb, int ntiles, int geo, hipStream_t s);
