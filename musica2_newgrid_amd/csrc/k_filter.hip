@@ -72,7 +72,7 @@ __device__ __forceinline__ void halo_setup(const Geom &g, int i0, int j0, Halo &
       h.on[s] = gj <= g.ny && gi <= g.nx + 5;
       h.r[s] = r;
       h.c[s] = li;
-      h.off[s] = lin(g, gi, gj, 0);
+      h.off[s] = lin_w(g, gi, gj);
     } else if (t < NH) {
       const int tt = t - NHX;
       const int r = tt / FX, c = tt % FX;
@@ -82,7 +82,7 @@ __device__ __forceinline__ void halo_setup(const Geom &g, int i0, int j0, Halo &
       h.xdir[s] = false;
       h.r[s] = lj;
       h.c[s] = c;
-      h.off[s] = lin(g, gi, gj, 0);
+      h.off[s] = lin_w(g, gi, gj);
     }
   }
 }
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(FT, 2) void k_filter_sf(const Batch<FilterArgs> *__
   const int i = i0 + tx, j = j0 + ty;
   const bool own = i <= g.nx && j <= g.ny;
   const bool needx = i <= g.nx + 5 && j <= g.ny, needy = i <= g.nx && j <= g.ny + 5;
-  const idx_t sz = g.sy, own_off = lin(g, i, j, 0);
+  const idx_t sz = g.sy, own_off = lin_w(g, i, j);
   Halo hl;
   halo_setup(g, i0, j0, hl);
   R dd[6];
@@ -147,14 +147,14 @@ __global__ __launch_bounds__(FT, 2) void k_filter_sf(const Batch<FilterArgs> *__
   R q[11][5];
   if (own) {
 #pragma unroll
-    for (int l = 0; l < 10; l++) ldr(uinp, own_off + (idx_t)(kbeg - 5 + l) * sz, q[l]);
+    for (int l = 0; l < 10; l++) ldr(uinp, own_off + (idx_t)wrap_k(g, kbeg - 5 + l) * sz, q[l]);
   }
   // the state loads of a plane (queue point k+5, pencil cell, halo cells)
   // are issued one plane ahead, during the previous plane's stencils
   R qn[5], uc[5], uh[NS][5];
   {
     const idx_t pk = own_off + (idx_t)kbeg * sz;
-    if (own) ldr(uinp, pk + 5 * sz, qn);
+    if (own) ldr(uinp, own_off + (idx_t)wrap_k(g, kbeg + 5) * sz, qn);
     if (!own && (needx || needy)) ldr(uinp, pk, uc);
 #pragma unroll
     for (int s = 0; s < NS; s++)
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(FT, 2) void k_filter_sf(const Batch<FilterArgs> *__
     __syncthreads();
     if (k < kend) {
       const idx_t pn = pk + sz;
-      if (own) ldr(uinp, pn + 5 * sz, qn);
+      if (own) ldr(uinp, own_off + (idx_t)wrap_k(g, k + 6) * sz, qn);
       if (!own && (needx || needy)) ldr(uinp, pn, uc);
 #pragma unroll
       for (int s = 0; s < NS; s++)
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(FT, 2) void k_filter_shock(const Batch<FilterArgs> 
   const bool needx = i <= g.nx + 5 && j <= g.ny, needy = i <= g.nx && j <= g.ny + 5;
   const bool duc = !ARTV && a.sens != nullptr;
   const double cs = a.csens;
-  const idx_t sz = g.sy, own_off = lin(g, i, j, 0);
+  const idx_t sz = g.sy, own_off = lin_w(g, i, j);
   Halo hl;
   halo_setup(g, i0, j0, hl);
   // p / sensor cells of this thread: rows of spx (i-direction) then of spy
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(FT, 2) void k_filter_shock(const Batch<FilterArgs> 
       pp_s[s] = c >= 1 && c <= FX + 2 && gi <= g.nx + 1;  // sensor needed at i0-1..i0+FX
       pp_r[s] = r;
       pp_c[s] = c;
-      pp_off[s] = lin(g, gi, gj, 0);
+      pp_off[s] = lin_w(g, gi, gj);
     } else if (t < NPX + NPY) {
       const int tt = t - NPX;
       const int r = tt / FX, c = tt % FX;
@@ -360,7 +360,7 @@ __global__ __launch_bounds__(FT, 2) void k_filter_shock(const Batch<FilterArgs> 
       pp_x[s] = false;
       pp_r[s] = r;
       pp_c[s] = c;
-      pp_off[s] = lin(g, gi, gj, 0);
+      pp_off[s] = lin_w(g, gi, gj);
     }
   }
 
@@ -369,16 +369,16 @@ __global__ __launch_bounds__(FT, 2) void k_filter_shock(const Batch<FilterArgs> 
   double qs[3];      // sensor at k-1..k+1
   if (own) {
 #pragma unroll
-    for (int l = 0; l < 10; l++) ldr(uinp, own_off + (idx_t)(kbeg - 5 + l) * sz, q[l]);
+    for (int l = 0; l < 10; l++) ldr(uinp, own_off + (idx_t)wrap_k(g, kbeg - 5 + l) * sz, q[l]);
     if constexpr (ARTV) {
 #pragma unroll
-      for (int l = 0; l < 2; l++) qp[l] = ldg(prsp, own_off + (idx_t)(kbeg - 1 + l) * sz);
+      for (int l = 0; l < 2; l++) qp[l] = ldg(prsp, own_off + (idx_t)wrap_k(g, kbeg - 1 + l) * sz);
     } else {
 #pragma unroll
-      for (int l = 0; l < 4; l++) qp[l] = ldg(prsp, own_off + (idx_t)(kbeg - 2 + l) * sz);
+      for (int l = 0; l < 4; l++) qp[l] = ldg(prsp, own_off + (idx_t)wrap_k(g, kbeg - 2 + l) * sz);
     }
 #pragma unroll
-    for (int l = 0; l < 2; l++) qs[l] = duc ? ldg(sensp, own_off + (idx_t)(kbeg - 1 + l) * sz) : 1.0;
+    for (int l = 0; l < 2; l++) qs[l] = duc ? ldg(sensp, own_off + (idx_t)wrap_k(g, kbeg - 1 + l) * sz) : 1.0;
   }
 
   // every global load of a plane is issued one plane ahead, during the
@@ -388,9 +388,10 @@ __global__ __launch_bounds__(FT, 2) void k_filter_shock(const Batch<FilterArgs> 
   auto load_plane = [&](int kk) {
     const idx_t pkk = own_off + (idx_t)kk * sz;
     if (own) {
-      ldr(uinp, pkk + 5 * sz, qn);
-      qpn = ARTV ? ldg(prsp, pkk + sz) : ldg(prsp, pkk + 2 * sz);
-      qsn = duc ? ldg(sensp, pkk + sz) : 1.0;
+      const idx_t p1 = own_off + (idx_t)wrap_k(g, kk + 1) * sz;
+      ldr(uinp, own_off + (idx_t)wrap_k(g, kk + 5) * sz, qn);
+      qpn = ARTV ? ldg(prsp, p1) : ldg(prsp, own_off + (idx_t)wrap_k(g, kk + 2) * sz);
+      qsn = duc ? ldg(sensp, p1) : 1.0;
     }
     if (!own && (needx || needy)) ldr(uinp, pkk, uc);
 #pragma unroll

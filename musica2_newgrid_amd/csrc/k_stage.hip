@@ -46,8 +46,18 @@ struct Prim {
   double r, ru, rv, rw, re, u, v, w, pr;
 };
 
+__device__ __forceinline__ double d11_terms(double d1, double d2, double d3, double d4, double d5) {
+#pragma clang fp contract(off)
+  return __builtin_fma(
+      A11_5, d5,
+      __builtin_fma(A11_4, d4, __builtin_fma(A11_3, d3, __builtin_fma(A11_1, d1, A11_2 * d2))));
+}
+
 template <class R>
 __device__ __forceinline__ R d11c(const R *f, int s) {
+  if constexpr (std::is_same<R, double>::value)
+    return d11_terms(f[s] - f[-s], f[2 * s] - f[-2 * s], f[3 * s] - f[-3 * s], f[4 * s] - f[-4 * s],
+                     f[5 * s] - f[-5 * s]);
   return R(A11_1) * (f[s] - f[-s]) + R(A11_2) * (f[2 * s] - f[-2 * s]) + R(A11_3) * (f[3 * s] - f[-3 * s]) +
          R(A11_4) * (f[4 * s] - f[-4 * s]) + R(A11_5) * (f[5 * s] - f[-5 * s]);
 }
@@ -149,17 +159,19 @@ __device__ __forceinline__ void load_u(const Ptrs &P, idx_t p, double u[5]) {
   }
 }
 
+// State at element p, metrics at element pm (a wrapped axis: the state at the
+// periodic image, the metrics at the point itself, as the caller gave them).
 // The flux-direction metric terms are read as FP32 in the mixed path (its
 // flux arithmetic rounds them to FP32 anyway: the same values, half the
 // bytes), as FP64 otherwise.
 template <bool CURV, bool IN32, bool MIX>
-__device__ __forceinline__ void load_raw(const Ptrs &P, idx_t p, int dir, Raw &r) {
+__device__ __forceinline__ void load_raw(const Ptrs &P, idx_t p, idx_t pm, int dir, Raw &r) {
   load_u<IN32>(P, p, r.u);
   if constexpr (CURV) {
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      if constexpr (MIX) r.m[c] = (double)ldg(P.m32[3 * dir + c], p);
-      else r.m[c] = ldg(P.m[3 * dir + c], p);
+      if constexpr (MIX) r.m[c] = (double)ldg(P.m32[3 * dir + c], pm);
+      else r.m[c] = ldg(P.m[3 * dir + c], pm);
     }
   }
 }
@@ -167,9 +179,9 @@ __device__ __forceinline__ void load_raw(const Ptrs &P, idx_t p, int dir, Raw &r
 // Raw inputs of a halo cell, whose direction is known at run time only:
 // branch to a constant direction so that the pointer table stays in registers.
 template <bool CURV, bool IN32, bool MIX>
-__device__ __forceinline__ void load_raw_halo(const Ptrs &P, idx_t p, int dir, Raw &r) {
-  if (dir == 0) load_raw<CURV, IN32, MIX>(P, p, 0, r);
-  else load_raw<CURV, IN32, MIX>(P, p, 1, r);
+__device__ __forceinline__ void load_raw_halo(const Ptrs &P, idx_t p, idx_t pm, int dir, Raw &r) {
+  if (dir == 0) load_raw<CURV, IN32, MIX>(P, p, pm, 0, r);
+  else load_raw<CURV, IN32, MIX>(P, p, pm, 1, r);
 }
 
 __device__ __forceinline__ Prim prim_raw(const double u[5], double gam1) {
@@ -249,6 +261,48 @@ __device__ __forceinline__ void flux_r(const Prim &q, int dir, const double m[3]
   else flux_m<CURV>(q, dir, m, F);
 }
 
+// The FP64 arithmetic of 3-D curvilinear blocks with its roundings written
+// out: left to the compiler, which product of a sum is fused depends on the
+// code around it, and where a variable is small beside the terms that cancel
+// in it (the transverse momentum ahead of a pulse in a uniform stream, 1e-9
+// of the stream's) results of two builds, tile shapes or variants differ in
+// the digits that carry it.  t = rho E - rho |u|^2 / 2, so that p = gam1 t.
+struct PrimC3 {
+  double r, re, u, v, w, t, pr;
+};
+__device__ __forceinline__ PrimC3 prim_c3(const double U[5], double gam1) {
+#pragma clang fp contract(off)
+  PrimC3 q;
+  q.r = U[0];
+  q.re = U[4];
+  const double vi = 1.0 / q.r;
+  q.u = U[1] * vi;
+  q.v = U[2] * vi;
+  q.w = U[3] * vi;
+  const double s = __builtin_fma(q.w, q.w, __builtin_fma(q.u, q.u, q.v * q.v));
+  q.t = __builtin_fma(-0.5 * q.r, s, q.re);
+  q.pr = gam1 * q.t;
+  return q;
+}
+// SITE: kOwn, the i- and j-fluxes of the thread's own point; kQueue, its
+// k-flux and the first halo cell; kHalo, the further halo cells.
+enum FluxSite { kQueue, kOwn, kHalo };
+template <FluxSite SITE>
+__device__ __forceinline__ void flux_c3(const PrimC3 &q, double gam1, const double m[3], double F[5]) {
+#pragma clang fp contract(off)
+  const double vc = __builtin_fma(q.w, m[2], __builtin_fma(q.u, m[0], q.v * m[1]));
+  const double rovc = q.r * vc;
+  const double u[3] = {q.u, q.v, q.w};
+  F[0] = rovc;
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    if constexpr (SITE == kHalo) F[1 + c] = __builtin_fma(u[c], rovc, m[c] * q.pr);
+    else F[1 + c] = __builtin_fma(m[c], q.pr, u[c] * rovc);
+  }
+  if constexpr (SITE == kOwn) F[4] = (q.re + q.pr) * vc;
+  else F[4] = __builtin_fma(gam1, q.t, q.re) * vc;
+}
+
 // Flux of a halo cell, whose direction (i or j) is only known at run time:
 // branch to a constant direction so that the primitives stay in registers.
 template <bool CURV, bool MIX, class R>
@@ -281,6 +335,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
   constexpr bool IBND = WALL && !CURV;
   constexpr bool ADV = WALL == 2;
   constexpr bool MIX = MODE != kFP64;
+  constexpr bool PIN = C3 && !MIX && !WALL;  // roundings written out (flux_c3)
   constexpr bool IN32 = MODE == kMixMiddle || MODE == kMixLast;
   constexpr bool OUT32 = MODE == kMixFirst || MODE == kMixMiddle;
   using R = typename std::conditional<MIX, float, double>::type;
@@ -318,7 +373,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
 
   // halo cells handled by this thread: LDS slot, padded offset in the plane, direction
   int hs_dir[NS], hs_r[NS], hs_c[NS];
-  idx_t hs_off[NS];
+  idx_t hs_off[NS], hs_moff[NS];  // state, metrics
   bool hs_on[NS];
 #pragma unroll
   for (int s = 0; s < NS; s++) {
@@ -326,7 +381,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
     hs_on[s] = false;
     hs_dir[s] = 0;
     hs_r[s] = hs_c[s] = 0;
-    hs_off[s] = 0;
+    hs_off[s] = hs_moff[s] = 0;
     if (h < NHX) {
       const int r = h / 10, c = h % 10;
       const int li = c < 5 ? c : TX + c;
@@ -335,7 +390,8 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
       hs_dir[s] = 0;
       hs_r[s] = r;
       hs_c[s] = li;
-      hs_off[s] = lin(g, gi, gj, 0);
+      hs_moff[s] = lin(g, gi, gj, 0);
+      hs_off[s] = WALL ? hs_moff[s] : lin_w(g, gi, gj);
     } else if (h < NH) {
       const int hh = h - NHX;
       const int r = hh / TX, c = hh % TX;
@@ -345,10 +401,12 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
       hs_dir[s] = 1;
       hs_r[s] = lj;
       hs_c[s] = c;
-      hs_off[s] = lin(g, gi, gj, 0);
+      hs_moff[s] = lin(g, gi, gj, 0);
+      hs_off[s] = WALL ? hs_moff[s] : lin_w(g, gi, gj);
     }
   }
-  idx_t own_off = lin(g, i, j, 0);
+  const idx_t own_moff = lin(g, i, j, 0);
+  idx_t own_off = WALL ? own_moff : lin_w(g, i, j);
   const idx_t sz = g.sy;
   // 2.5-D: the metric rows of the halo cells and of the own column, and
   // 1/J, constant along k: loaded once
@@ -360,7 +418,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
     for (int s = 0; s < NS; s++) {
       hm[s][0] = hm[s][1] = 0.0;
       if (hs_on[s]) {
-        const idx_t p2 = hs_off[s] - (idx_t)(G - 1) * sz;  // the cell's (i, j) column
+        const idx_t p2 = hs_moff[s] - (idx_t)(G - 1) * sz;  // the cell's (i, j) column
         // (constant indices only: a run-time index would move the pointer table to scratch)
         const bool xd = hs_dir[s] == 0;
         hm[s][0] = ldg(xd ? P.m2[0] : P.m2[2], p2);
@@ -464,6 +522,8 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
     for (int s = 0; s < NS; s++) hs_beyond[s] = false;
   }
 
+  // (a case with boundary faces does not wrap: one offset serves both)
+  auto kwrap = [&](int k) { return WALL ? k : wrap_k(g, k); };
   const RefState &rf = a.ref;
   const double alpha = a.alpha;
   R q[11][5];
@@ -475,15 +535,17 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
 #pragma unroll
     for (int l = 0; l < 10; l++) {
       Raw r;
-      load_raw<C3, IN32, MIX>(P, own_off + (idx_t)(kbeg - 5 + l) * sz, 2, r);
-      flux_r<C3, MIX>(prim_raw(r.u, gam1), 2, r.m, rf, q[l]);
+      load_raw<C3, IN32, MIX>(P, own_off + (idx_t)kwrap(kbeg - 5 + l) * sz, (WALL ? own_off : own_moff) + (idx_t)(kbeg - 5 + l) * sz, 2, r);
+      if constexpr (PIN) flux_c3<kQueue>(prim_c3(r.u, gam1), gam1, r.m, q[l]);
+      else flux_r<C3, MIX>(prim_raw(r.u, gam1), 2, r.m, rf, q[l]);
     }
-    load_raw<C3, IN32, MIX>(P, own_off + (idx_t)(kbeg + 5) * sz, 2, rq);
+    load_raw<C3, IN32, MIX>(P, own_off + (idx_t)kwrap(kbeg + 5) * sz, (WALL ? own_off : own_moff) + (idx_t)(kbeg + 5) * sz, 2, rq);
   }
   // the own point's state and (c3) i/j metric terms, likewise one plane ahead
   double ru[5] = {0, 0, 0, 0, 0};
-  auto load_own = [&](idx_t p) {
-    load_u<IN32>(P, p, ru);
+  auto load_own = [&](int kk) {
+    load_u<IN32>(P, own_off + (idx_t)kk * sz, ru);
+    const idx_t p = (WALL ? own_off : own_moff) + (idx_t)kk * sz;
     if constexpr (C3) {
 #pragma unroll
       for (int c = 0; c < 3; c++) {
@@ -492,7 +554,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
       }
     }
   };
-  if (needx || needy) load_own(own_off + (idx_t)kbeg * sz);
+  if (needx || needy) load_own(kbeg);
 
   for (int k = kbeg; k <= kend; k++) {
     const idx_t pk = own_off + (idx_t)k * sz;
@@ -502,7 +564,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
     Raw rh0;
     double u0[5] = {0, 0, 0, 0, 0};
     if (hs_on[0]) {
-      load_raw_halo<C3, IN32, MIX>(P, hs_off[0] + (idx_t)k * sz, hs_dir[0], rh0);
+      load_raw_halo<C3, IN32, MIX>(P, hs_off[0] + (idx_t)k * sz, (WALL ? hs_off[0] : hs_moff[0]) + (idx_t)k * sz, hs_dir[0], rh0);
       if constexpr (C2) {
         rh0.m[0] = hm[0][0];
         rh0.m[1] = hm[0][1];
@@ -519,9 +581,15 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
         for (int c = 0; c < 4; c++) kvis[c] = ldg_nt(P.kv[c], pk);
       }
     }
-    if (own) flux_r<C3, MIX>(prim_raw(rq.u, gam1), 2, rq.m, rf, q[10]);
+    if (own) {
+      if constexpr (PIN) flux_c3<kQueue>(prim_c3(rq.u, gam1), gam1, rq.m, q[10]);
+      else flux_r<C3, MIX>(prim_raw(rq.u, gam1), 2, rq.m, rf, q[10]);
+    }
     if (needx || needy) {
-      const Prim pq = prim_raw(ru, gam1);
+      Prim pq;
+      PrimC3 pc;
+      if constexpr (PIN) pc = prim_c3(ru, gam1);
+      else pq = prim_raw(ru, gam1);
       R F[5];
       if (needx) {
         if (IBND && i == 1 && P.uin_row) {
@@ -539,6 +607,8 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
           pi.rw = ldg(P.uin_row, 3 * ss + sl);
           pi.re = ldg(P.uin_row, 4 * ss + sl);
           flux_r<CURV, MIX>(pi, 0, rxm, rf, F);
+        } else if constexpr (PIN) {
+          flux_c3<kOwn>(pc, gam1, rxm, F);
         } else {
           flux_r<CURV, MIX>(pq, 0, rxm, rf, F);
         }
@@ -547,7 +617,8 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
           sfx[v][ty][tx + 5] = ADV ? pencil_value(acode >> 30, F[v]) : ((IBND && own_beyond_x) ? R(0) : F[v]);
       }
       if (needy) {
-        flux_r<CURV, MIX>(pq, 1, rym, rf, F);
+        if constexpr (PIN) flux_c3<kOwn>(pc, gam1, rym, F);
+        else flux_r<CURV, MIX>(pq, 1, rym, rf, F);
 #pragma unroll
         for (int v = 0; v < 5; v++)
           sfy[v][ty + 5][tx] = ADV ? pencil_value((acode >> 28) & 3u, F[v]) : ((WALL && own_beyond) ? R(0) : F[v]);
@@ -555,7 +626,8 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
     }
     if (hs_on[0]) {
       R F[5];
-      flux_halo<CURV, MIX>(prim_raw(rh0.u, gam1), hs_dir[0], rh0.m, rf, F);
+      if constexpr (PIN) flux_c3<kQueue>(prim_c3(rh0.u, gam1), gam1, rh0.m, F);
+      else flux_halo<CURV, MIX>(prim_raw(rh0.u, gam1), hs_dir[0], rh0.m, rf, F);
       if (hs_dir[0] == 0) {
 #pragma unroll
         for (int v = 0; v < 5; v++)
@@ -573,7 +645,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
 #pragma unroll
       for (int s = 1; s < NS; s++)
         if (hs_on[s]) {
-          load_raw_halo<C3, IN32, MIX>(P, hs_off[s] + (idx_t)k * sz, hs_dir[s], rh[s]);
+          load_raw_halo<C3, IN32, MIX>(P, hs_off[s] + (idx_t)k * sz, (WALL ? hs_off[s] : hs_moff[s]) + (idx_t)k * sz, hs_dir[s], rh[s]);
           if constexpr (C2) {
             rh[s].m[0] = hm[s][0];
             rh[s].m[1] = hm[s][1];
@@ -584,7 +656,8 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
       for (int s = 1; s < NS; s++) {
         if (hs_on[s]) {
           R F[5];
-          flux_halo<CURV, MIX>(prim_raw(rh[s].u, gam1), hs_dir[s], rh[s].m, rf, F);
+          if constexpr (PIN) flux_c3<kHalo>(prim_c3(rh[s].u, gam1), gam1, rh[s].m, F);
+          else flux_halo<CURV, MIX>(prim_raw(rh[s].u, gam1), hs_dir[s], rh[s].m, rf, F);
           if (hs_dir[s] == 0) {
 #pragma unroll
             for (int v = 0; v < 5; v++)
@@ -601,8 +674,8 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
     }
     __syncthreads();
     // queue point and own point of the next plane
-    if (own && k < kend) load_raw<C3, IN32, MIX>(P, pk + 6 * sz, 2, rq);
-    if ((needx || needy) && k < kend) load_own(pk + sz);
+    if (own && k < kend) load_raw<C3, IN32, MIX>(P, own_off + (idx_t)kwrap(k + 6) * sz, (WALL ? own_off : own_moff) + (idx_t)k * sz + 6 * sz, 2, rq);
+    if ((needx || needy) && k < kend) load_own(k + 1);
 
     if (own) {
       double K[5];
@@ -624,12 +697,17 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
         } else {
           dy = d11c(&sfy[v][ty + 5][tx], TX);
         }
-        const R dz = R(A11_1) * (q[6][v] - q[4][v]) + R(A11_2) * (q[7][v] - q[3][v]) +
-                     R(A11_3) * (q[8][v] - q[2][v]) + R(A11_4) * (q[9][v] - q[1][v]) +
-                     R(A11_5) * (q[10][v] - q[0][v]);
+        R dz;
+        if constexpr (MIX)
+          dz = R(A11_1) * (q[6][v] - q[4][v]) + R(A11_2) * (q[7][v] - q[3][v]) + R(A11_3) * (q[8][v] - q[2][v]) +
+               R(A11_4) * (q[9][v] - q[1][v]) + R(A11_5) * (q[10][v] - q[0][v]);
+        else
+          dz = d11_terms(q[6][v] - q[4][v], q[7][v] - q[3][v], q[8][v] - q[2][v], q[9][v] - q[1][v],
+                         q[10][v] - q[0][v]);
         // metrics and Jacobian multiply in FP64
         if constexpr (C3) {
-          K[v] = (double)(dz + (dy + dx)) * ijac;
+          if constexpr (PIN && VISC) K[v] = v ? __builtin_fma(dz + (dy + dx), ijac, kvis[v ? v - 1 : 0]) : (dz + (dy + dx)) * ijac;
+          else K[v] = (double)(dz + (dy + dx)) * ijac;
         } else if constexpr (C2) {
           // (ksi + eta parts) * ijacob, then the Cartesian z part
           K[v] = (double)dz * ldg(P.idz, (idx_t)(k - 1 + G)) + (double)(dy + dx) * ijac;
@@ -662,7 +740,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const Batch<StageArgs> *__r
           }
         }
       }
-      if constexpr (VISC) {
+      if constexpr (VISC && !PIN) {
         if (!kslab) {
 #pragma unroll
           for (int c = 0; c < 4; c++) K[1 + c] = K[1 + c] + kvis[c];
@@ -785,7 +863,7 @@ struct DmaLane {
 };
 
 template <int TX, int TY, int EW>
-__device__ __forceinline__ void dma_lane(const Geom &g, int i0, int j0, int lane, DmaLane<TX, TY, EW> &L) {
+__device__ __forceinline__ void dma_lane(const Geom &g, int i0, int j0, int lane, bool wrap, DmaLane<TX, TY, EW> &L) {
   using D = DmaPlan<TX, TY, EW>;
   using HM = HaloMap<TX, TY>;
   const idx_t org = lin(g, i0, j0, 0);
@@ -806,7 +884,7 @@ __device__ __forceinline__ void dma_lane(const Geom &g, int i0, int j0, int lane
       bool ok, jd;
       HM::cell(h, i0, j0, g, gi, gj, ok, jd, pr, pc);
       if (ok) {
-        off = lin(g, gi, gj, 0);
+        off = wrap ? lin_w(g, gi, gj) : lin(g, gi, gj, 0);
         extra = (uint32_t)(part * 4);
       }
     }
@@ -818,7 +896,8 @@ __device__ __forceinline__ void dma_lane(const Geom &g, int i0, int j0, int lane
 // arrays the j-halo / i-halo read (wave-uniform), dst the LDS image.
 template <int TX, int TY, int EW>
 __device__ __forceinline__ void dma_issue(const MGPU_GLOBAL char *bj, const MGPU_GLOBAL char *bi, void *dst,
-                                          const DmaLane<TX, TY, EW> &L, const Geom &g, int i0, int j0, int lane) {
+                                          const DmaLane<TX, TY, EW> &L, const Geom &g, int i0, int j0, int lane,
+                                          bool wrap) {
   using D = DmaPlan<TX, TY, EW>;
   uint32_t *ldst = reinterpret_cast<uint32_t *>(dst);
 #pragma unroll
@@ -826,7 +905,7 @@ __device__ __forceinline__ void dma_issue(const MGPU_GLOBAL char *bj, const MGPU
     const int lj = r < 5 ? r : TY + r;
     const int gj = j0 - 5 + lj;
     if (gj > g.ny + 5) continue;  // beyond the valid region: nothing reads this row
-    const MGPU_GLOBAL char *row = bj + (uint32_t)(lin(g, i0, gj, 0) * (idx_t)(4 * EW));
+    const MGPU_GLOBAL char *row = bj + (uint32_t)((wrap ? lin_w(g, i0, gj) : lin(g, i0, gj, 0)) * (idx_t)(4 * EW));
 #pragma unroll
     for (int p = 0; p < D::R; p++) {
       lds_void_t *l = (lds_void_t *)(ldst + r * D::RW + 64 * p);
@@ -906,7 +985,7 @@ __global__ __launch_bounds__(TX *TY, 1) void k_stage_p(const Batch<StageArgs> *_
         hs_beyond[s] = hs_jd[s] && (((g.jbnd & 1) && gj < 1) || ((g.jbnd & 2) && gj > g.ny));
     }
   }
-  const idx_t own_off = lin(g, i, j, 0);
+  const idx_t own_off = lin_w(g, i, j), own_moff = lin(g, i, j, 0);
   // 2.5-D: metric rows of the halo cells and the own column, 1/J (constant in k)
   double hm[NS][2];
   double rxm[3] = {0, 0, 0}, rym[3] = {0, 0, 0};
@@ -960,7 +1039,7 @@ __global__ __launch_bounds__(TX *TY, 1) void k_stage_p(const Batch<StageArgs> *_
         else src = P.uin[q];
       }
     dbj = dbi = reinterpret_cast<const MGPU_GLOBAL char *>((const MGPU_GLOBAL TU *)src);
-    dma_lane<TX, TY, EWU>(g, i0, j0, lane, dlu);
+    dma_lane<TX, TY, EWU>(g, i0, j0, lane, true, dlu);
   } else if (dmet) {
     if constexpr (C3) {
 #pragma unroll
@@ -969,7 +1048,7 @@ __global__ __launch_bounds__(TX *TY, 1) void k_stage_p(const Batch<StageArgs> *_
           dbi = reinterpret_cast<const MGPU_GLOBAL char *>((const MGPU_GLOBAL double *)P.m[c]);
           dbj = reinterpret_cast<const MGPU_GLOBAL char *>((const MGPU_GLOBAL double *)P.m[3 + c]);
         }
-      dma_lane<TX, TY, 2>(g, i0, j0, lane, dlm);
+      dma_lane<TX, TY, 2>(g, i0, j0, lane, false, dlm);
     }
   }
   auto dma = [&](int k, int b) {
@@ -977,13 +1056,13 @@ __global__ __launch_bounds__(TX *TY, 1) void k_stage_p(const Batch<StageArgs> *_
       const uint32_t kb = (uint32_t)((idx_t)k * sz * (idx_t)sizeof(TU));
 #pragma unroll
       for (int q = 0; q < 5; q++)
-        if (q == wv) dma_issue<TX, TY, EWU>(dbj + kb, dbi + kb, &hu[b][q][0], dlu, g, i0, j0, lane);
+        if (q == wv) dma_issue<TX, TY, EWU>(dbj + kb, dbi + kb, &hu[b][q][0], dlu, g, i0, j0, lane, true);
     } else if (dmet) {
       if constexpr (C3) {
         const uint32_t kb = (uint32_t)((idx_t)k * sz * (idx_t)sizeof(double));
 #pragma unroll
         for (int c = 0; c < NM; c++)
-          if (c == wv - 5) dma_issue<TX, TY, 2>(dbj + kb, dbi + kb, &hmt[b][c][0], dlm, g, i0, j0, lane);
+          if (c == wv - 5) dma_issue<TX, TY, 2>(dbj + kb, dbi + kb, &hmt[b][c][0], dlm, g, i0, j0, lane, false);
       }
     }
   };
@@ -997,14 +1076,15 @@ __global__ __launch_bounds__(TX *TY, 1) void k_stage_p(const Batch<StageArgs> *_
 #pragma unroll
     for (int l = 0; l < 10; l++) {
       Raw r;
-      load_raw<C3, IN32, MIX>(P, own_off + (idx_t)(kbeg - 5 + l) * sz, 2, r);
+      load_raw<C3, IN32, MIX>(P, own_off + (idx_t)wrap_k(g, kbeg - 5 + l) * sz, own_moff + (idx_t)(kbeg - 5 + l) * sz, 2, r);
       flux_r<C3, MIX>(prim_raw(r.u, gam1), 2, r.m, rf, q[l]);
     }
-    load_raw<C3, IN32, MIX>(P, own_off + (idx_t)(kbeg + 5) * sz, 2, rq);
+    load_raw<C3, IN32, MIX>(P, own_off + (idx_t)wrap_k(g, kbeg + 5) * sz, own_moff + (idx_t)(kbeg + 5) * sz, 2, rq);
   }
   double ru[5] = {0, 0, 0, 0, 0};
-  auto load_own = [&](idx_t p) {
-    load_u<IN32>(P, p, ru);
+  auto load_own = [&](int kk) {
+    load_u<IN32>(P, own_off + (idx_t)kk * sz, ru);
+    const idx_t p = (WALL ? own_off : own_moff) + (idx_t)kk * sz;
     if constexpr (C3) {
 #pragma unroll
       for (int c = 0; c < 3; c++) {
@@ -1013,7 +1093,7 @@ __global__ __launch_bounds__(TX *TY, 1) void k_stage_p(const Batch<StageArgs> *_
       }
     }
   };
-  if (needx || needy) load_own(own_off + (idx_t)kbeg * sz);
+  if (needx || needy) load_own(kbeg);
   // U^n, 1/J (c3) and K_v of the own point, one plane ahead like the rest
   // (Cartesian and 2.5-D: idz of the plane; the own column's idx and idy
   // are constant along the march)
@@ -1138,10 +1218,10 @@ __global__ __launch_bounds__(TX *TY, 1) void k_stage_p(const Batch<StageArgs> *_
     barrier_lds();
     // own point and queue point of plane k+1, in flight during the derivatives
     if (own && k < kend) {
-      load_raw<C3, IN32, MIX>(P, pk + 6 * sz, 2, rq);
+      load_raw<C3, IN32, MIX>(P, own_off + (idx_t)wrap_k(g, k + 6) * sz, pk + 6 * sz, 2, rq);
       load_u0(pk + sz, k + 1);
     }
-    if ((needx || needy) && k < kend) load_own(pk + sz);
+    if ((needx || needy) && k < kend) load_own(k + 1);
 
     if (own) {
       double K[5];

@@ -111,7 +111,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_visc(const Batch<ViscArgs> *__res
       hs_on[s] = gj <= g.ny && gi <= g.nx + 2;
       hs_r[s] = r;
       hs_c[s] = li;
-      hs_off[s] = lin(g, gi, gj, 0);
+      hs_off[s] = lin_w(g, gi, gj);
     } else if (h < NH) {
       const int hh = h - NHX;
       const int r = hh / TX, c = hh % TX;
@@ -121,10 +121,10 @@ __global__ __launch_bounds__(TX *TY, 2) void k_visc(const Batch<ViscArgs> *__res
       hs_dir[s] = 1;
       hs_r[s] = lj;
       hs_c[s] = c;
-      hs_off[s] = lin(g, gi, gj, 0);
+      hs_off[s] = lin_w(g, gi, gj);
     }
   }
-  const idx_t own_off = lin(g, i, j, 0);
+  const idx_t own_off = lin_w(g, i, j);
   // 2.5-D: the column's viscous metrics (y_eta, -x_eta, -y_ksi, x_ksi, ijacob),
   // the same in every plane
   double mc2[5] = {0, 0, 0, 0, 0};
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_visc(const Batch<ViscArgs> *__res
 #pragma unroll
     for (int l = 0; l < 4; l++) {
       double U[5];
-      ld5(u0p, own_off + (idx_t)(kbeg - 2 + l) * sz, U);
+      ld5(u0p, own_off + (idx_t)wrap_k(g, kbeg - 2 + l) * sz, U);
       q[l] = prim5r(U, gam1, rg);
     }
   }
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_visc(const Batch<ViscArgs> *__res
     const idx_t pk = own_off + (idx_t)k * sz;
     // ---- every global load of the plane ----
     double uq[5], uc[5], uh[NS][5], mvv[10];
-    if (own) ld5(u0p, pk + 2 * sz, uq);
+    if (own) ld5(u0p, own_off + (idx_t)wrap_k(g, k + 2) * sz, uq);
     if (!own && (needx || needy)) ld5(u0p, pk, uc);
 #pragma unroll
     for (int s = 0; s < NS; s++)
@@ -398,11 +398,11 @@ __global__ __launch_bounds__(TX *TY, 2) void k_vdiv(const Batch<VdivArgs> *__res
   const int kend = min(kbeg + kchunk - 1, g.nz);
   const bool own = i <= g.nx && j <= g.ny;
   const bool needx = i <= g.nx + 2 && j <= g.ny, needy = i <= g.nx && j <= g.ny + 2;
-  const idx_t sz = g.sy, own_off = lin(g, i, j, 0);
+  const idx_t sz = g.sy, own_off = lin(g, i, j, 0), own_t = lin_w(g, i, j);
   const double *const *mv = mvp;
 
   int hs_r[NS], hs_c[NS];
-  idx_t hs_off[NS], hs_off2[NS];
+  idx_t hs_off[NS], hs_t[NS], hs_off2[NS];  // metrics; tau; 2-D metrics
   bool hs_on[NS], hs_x[NS];
 #pragma unroll
   for (int s = 0; s < NS; s++) {
@@ -410,7 +410,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_vdiv(const Batch<VdivArgs> *__res
     hs_on[s] = false;
     hs_x[s] = true;
     hs_r[s] = hs_c[s] = 0;
-    hs_off[s] = hs_off2[s] = 0;
+    hs_off[s] = hs_t[s] = hs_off2[s] = 0;
     if (h < NHX) {
       const int r = h / 4, c = h % 4;
       const int li = c < 2 ? c : TX + c;
@@ -419,6 +419,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_vdiv(const Batch<VdivArgs> *__res
       hs_r[s] = r;
       hs_c[s] = li;
       hs_off[s] = lin(g, gi, gj, 0);
+      hs_t[s] = lin_w(g, gi, gj);
       hs_off2[s] = lin2(g, gi, gj);
     } else if (h < NH) {
       const int hh = h - NHX;
@@ -430,6 +431,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_vdiv(const Batch<VdivArgs> *__res
       hs_r[s] = lj;
       hs_c[s] = c;
       hs_off[s] = lin(g, gi, gj, 0);
+      hs_t[s] = lin_w(g, gi, gj);
       hs_off2[s] = lin2(g, gi, gj);
     }
   }
@@ -458,15 +460,15 @@ __global__ __launch_bounds__(TX *TY, 2) void k_vdiv(const Batch<VdivArgs> *__res
       vflux<false>(t, 0.0, 0.0, 0.0, f);
     }
   };
-  // tau values of direction d at element p, projected into f[4]
-  auto flux_at = [&](int d, idx_t p, idx_t p2, double f[4]) {
+  // tau values of direction d at element pt, projected into f[4]
+  auto flux_at = [&](int d, idx_t pt, idx_t p, idx_t p2, double f[4]) {
     double t9[NTAU];
     if (CURV || (C2 && d < 2)) {
 #pragma unroll
-      for (int c = 0; c < NTAU; c++) t9[c] = ldg(taup[c], p);
+      for (int c = 0; c < NTAU; c++) t9[c] = ldg(taup[c], pt);
     } else {
 #pragma unroll
-      for (int c = 0; c < 4; c++) t9[krow(d, c)] = ldg(taup[krow(d, c)], p);
+      for (int c = 0; c < 4; c++) t9[krow(d, c)] = ldg(taup[krow(d, c)], pt);
     }
     proj(d, t9, p, p2, f);
   };
@@ -479,12 +481,13 @@ __global__ __launch_bounds__(TX *TY, 2) void k_vdiv(const Batch<VdivArgs> *__res
   double tw[3][NTAU];
   if (own) {
 #pragma unroll
-    for (int l = 0; l < 2; l++) flux_at(2, own_off + (idx_t)(kbeg - 2 + l) * sz, own_off2, q[l]);
+    for (int l = 0; l < 2; l++)
+      flux_at(2, own_t + (idx_t)wrap_k(g, kbeg - 2 + l) * sz, own_off + (idx_t)(kbeg - 2 + l) * sz, own_off2, q[l]);
 #pragma unroll
     for (int l = 0; l < 2; l++) {
-      const idx_t p = own_off + (idx_t)(kbeg + l) * sz;
+      const idx_t p = own_off + (idx_t)(kbeg + l) * sz, pt = own_t + (idx_t)wrap_k(g, kbeg + l) * sz;
 #pragma unroll
-      for (int c = 0; c < NTAU; c++) tw[l][c] = ldg(taup[c], p);
+      for (int c = 0; c < NTAU; c++) tw[l][c] = ldg(taup[c], pt);
       flux_of(2, tw[l], p, own_off2, q[2 + l]);
     }
   }
@@ -493,23 +496,25 @@ __global__ __launch_bounds__(TX *TY, 2) void k_vdiv(const Batch<VdivArgs> *__res
     double fx[4], fy[4], fh[NS][4];
     double ijv = 0.0;
     if (own) {
-      const idx_t p2 = pk + 2 * sz;
+      const idx_t p2 = pk + 2 * sz, pt = own_t + (idx_t)wrap_k(g, k + 2) * sz;
 #pragma unroll
-      for (int c = 0; c < NTAU; c++) tw[2][c] = ldg(taup[c], p2);
+      for (int c = 0; c < NTAU; c++) tw[2][c] = ldg(taup[c], pt);
       flux_of(2, tw[2], p2, own_off2, q[4]);
       if constexpr (CURV) ijv = ldg(mv[9], pk);
       if constexpr (C2) ijv = ldg(a.met.m2v[4], own_off2);
       flux_of(0, tw[0], pk, own_off2, fx);
       flux_of(1, tw[0], pk, own_off2, fy);
     } else {
-      if (needx) flux_at(0, pk, own_off2, fx);
-      if (needy) flux_at(1, pk, own_off2, fy);
+      const idx_t pt = own_t + (idx_t)k * sz;
+      if (needx) flux_at(0, pt, pk, own_off2, fx);
+      if (needy) flux_at(1, pt, pk, own_off2, fy);
     }
 #pragma unroll
     for (int s = 0; s < NS; s++)
       if (hs_on[s]) {
-        if (hs_x[s]) flux_at(0, hs_off[s] + (idx_t)k * sz, hs_off2[s], fh[s]);
-        else flux_at(1, hs_off[s] + (idx_t)k * sz, hs_off2[s], fh[s]);
+        const idx_t pt = hs_t[s] + (idx_t)k * sz, p = hs_off[s] + (idx_t)k * sz;
+        if (hs_x[s]) flux_at(0, pt, p, hs_off2[s], fh[s]);
+        else flux_at(1, pt, p, hs_off2[s], fh[s]);
       }
     if (needx) {
 #pragma unroll

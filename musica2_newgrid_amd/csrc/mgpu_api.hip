@@ -240,6 +240,41 @@ int exchange_state(mgpu_handle *h, int set) {
   return 0;
 }
 
+// The same inside a step: the faces of axes that wrap (Geom::wrap) have no
+// reader there.
+int exchange_inner(mgpu_handle *h, int set) {
+  ProfScope ps(h, MGPU_K_HALO);
+  IfaceArgs a = h->xs[set];
+  a.tasks = h->xi_tasks;
+  a.chunks = h->xi_chunks;
+  HIPCK(h, launch_iface(a, h->nchunks_i, h->stream));
+  return 0;
+}
+
+// Axis a of block b joins itself: both faces periodic, or interfaces with
+// the opposite face of the same block as they lie.
+bool self_joined(const mgpu_block &bl, int b, int a) {
+  for (int f = 2 * a; f < 2 * a + 2; f++) {
+    if (bl.face_kind[f] == MGPU_FACE_PERIODIC) continue;
+    if (bl.face_kind[f] != MGPU_FACE_INTERFACE || bl.nbr_block[f] != b || bl.nbr_face[f] != (f ^ 1) || bl.orient[f] != 0)
+      return false;
+  }
+  return true;
+}
+
+// Which axes wrap (Geom::wrap).  None in a case with boundary faces: there a
+// periodic ghost of a wall row holds the value from before bc_wall, which its
+// image no longer does; nor with the artificial viscosities, whose spectral
+// radii are read next to the point itself.
+void set_wrap(mgpu_handle *h) {
+  for (size_t b = 0; b < h->b.size(); b++) {
+    int w = 0;
+    if (!h->bnd && !is_artvisc(h->c))
+      for (int a = 0; a < 3; a++) w |= self_joined(h->blocks[b], (int)b, a) ? 1 << a : 0;
+    h->b[b].g.wrap = w;
+  }
+}
+
 // Neighbour of face f of block b: (block, face, orientation code).
 void face_nbr(const mgpu_block &bl, int b, int f, int &nb, int &nf, int &o) {
   if (bl.face_kind[f] == MGPU_FACE_PERIODIC) {
@@ -641,8 +676,9 @@ void face_vmap(const XSet &xs, int vb, int vn, const int dst_ax[3], const int sr
 // outside its arrays (a block table that passed check_topology never does)
 // or if, on a Cartesian case, a face's orientation does not meet the
 // neighbour's axes as the two blocks' axis relabelings say it must.
+// inner: without the faces of axes that wrap.
 bool build_tasks(const mgpu_case &c, const std::vector<BlockData> &bds, int ng, const XSet &xs,
-                 std::vector<FaceTask> &tasks, std::vector<IfaceChunk> &chunks) {
+                 std::vector<FaceTask> &tasks, std::vector<IfaceChunk> &chunks, bool inner = false) {
   tasks.clear();
   chunks.clear();
   for (int b = 0; b < c.nblocks; b++) {
@@ -650,7 +686,7 @@ bool build_tasks(const mgpu_case &c, const std::vector<BlockData> &bds, int ng, 
     const Geom &ga = bds[b].g;
     const int na[3] = {ga.nx, ga.ny, ga.nz};
     for (int f = 0; f < 6; f++) {
-      if (is_bound(A.face_kind[f])) continue;
+      if (is_bound(A.face_kind[f]) || (inner && (ga.wrap >> (f / 2) & 1))) continue;
       int nb, nf, o;
       face_nbr(A, b, f, nb, nf, o);
       const Geom &gb = bds[nb].g;
@@ -704,25 +740,27 @@ bool build_tasks(const mgpu_case &c, const std::vector<BlockData> &bds, int ng, 
   return true;
 }
 
-template <class T>
-int upload(mgpu_handle *h, const std::vector<T> &v, T **out) {
-  *out = nullptr;
-  if (v.empty()) return 0;
-  void *p = nullptr;
-  HIPCK(h, hipMalloc(&p, v.size() * sizeof(T)));
-  h->xtables.push_back(p);
-  HIPCK(h, hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
-  *out = (T *)p;
-  return 0;
-}
+// The exchange tables in one piece of device memory: the byte offset of each.
+struct TableImage {
+  std::vector<char> bytes;
+  template <class T>
+  size_t add(const std::vector<T> &v) {
+    const size_t off = (bytes.size() + 63) / 64 * 64;
+    bytes.resize(off + v.size() * sizeof(T));
+    if (!v.empty()) memcpy(bytes.data() + off, v.data(), v.size() * sizeof(T));
+    return off;
+  }
+};
 
 void free_exchange(mgpu_handle *h) {
-  for (void *p : h->xtables) (void)hipFree(p);
-  h->xtables.clear();
+  if (h->xtables) (void)hipFree(h->xtables);
+  h->xtables = nullptr;
   for (auto &x : h->xs) x = IfaceArgs{};
   for (auto &x : h->xf) x = IfaceArgs32{};
   h->xv = IfaceArgs{};
-  h->nchunks_s = h->nchunks_v = 0;
+  h->xi_tasks = nullptr;
+  h->xi_chunks = nullptr;
+  h->nchunks_s = h->nchunks_i = h->nchunks_v = 0;
   h->exchange_ready = false;
 }
 
@@ -734,6 +772,7 @@ int setup_exchange(mgpu_handle *h) {
   free_exchange(h);
   h->c.blocks = h->blocks.data();
   h->c.nblocks = (int)h->blocks.size();
+  set_wrap(h);
   if (h->b.empty()) {
     h->exchange_ready = true;
     return 0;
@@ -741,46 +780,48 @@ int setup_exchange(mgpu_handle *h) {
   std::vector<FaceTask> tasks;
   std::vector<IfaceChunk> chunks;
   const int nb = (int)h->b.size();
-  int rc;
+  TableImage img;
   // state: 5 layers, 5 variables, one pointer table per state set
   if (!build_tasks(h->c, h->b, G, XSet{}, tasks, chunks))
     return fail(h, MGPU_EINVAL,
                 "interface exchange would reach outside a block's arrays, or a face meets its neighbour's axes "
                 "otherwise than the blocks' axis relabelings require");
-  FaceTask *dt = nullptr;
-  IfaceChunk *dc = nullptr;
-  if ((rc = upload(h, tasks, &dt)) || (rc = upload(h, chunks, &dc))) return rc;
-  h->nchunks_s = (int)chunks.size();
+  const size_t o_st = img.add(tasks), o_sc = img.add(chunks);
+  const int ns = (int)chunks.size();
+  // inside a step: without the faces of axes that wrap
+  if (!build_tasks(h->c, h->b, G, XSet{}, tasks, chunks, true))
+    return fail(h, MGPU_EINVAL, "interface exchange would reach outside a block's arrays");
+  const size_t o_it = img.add(tasks), o_ic = img.add(chunks);
+  const int ni = (int)chunks.size();
+  size_t o_s[3], o_f[2] = {0, 0};
   for (int s = 0; s < 3; s++) {
     std::vector<double *> ptrs;
     for (int b = 0; b < nb; b++)
       for (int v = 0; v < 5; v++) ptrs.push_back(h->b[b].st[s][v]);
-    double **dp = nullptr;
-    if ((rc = upload(h, ptrs, &dp))) return rc;
-    h->xs[s] = IfaceArgs{dt, dc, dp, 5};
+    o_s[s] = img.add(ptrs);
   }
-  if (h->mixed) {
+  if (h->mixed)
     for (int s = 0; s < 2; s++) {
       std::vector<float *> ptrs;
       for (int b = 0; b < nb; b++)
         for (int v = 0; v < 5; v++) ptrs.push_back(h->b[b].sf[s][v]);
-      float **dp = nullptr;
-      if ((rc = upload(h, ptrs, &dp))) return rc;
-      h->xf[s] = IfaceArgs32{dt, dc, dp, 5};
+      o_f[s] = img.add(ptrs);
     }
-  }
   // viscous: 2 layers of tau (+ p and the sensor for the shock filter)
+  size_t o_vt = 0, o_vc = 0, o_v = 0;
+  int n_v = 0, nv = 0;
   if (h->c.iorder_visc) {
     const bool shock = has_sensor(h->c), artv = is_artvisc(h->c);
     XSet xv;
     xv.visc = true;
     xv.sensor = shock;
     xv.radii = artv;
-    const int nv = xv.nvar();
-    if (!build_tasks(h->c, h->b, 2, xv, tasks, chunks))
+    nv = xv.nvar();
+    if (!build_tasks(h->c, h->b, 2, xv, tasks, chunks, true))
       return fail(h, MGPU_EINVAL, "viscous interface exchange would reach outside a block's arrays");
-    if ((rc = upload(h, tasks, &dt)) || (rc = upload(h, chunks, &dc))) return rc;
-    h->nchunks_v = (int)chunks.size();
+    o_vt = img.add(tasks);
+    o_vc = img.add(chunks);
+    n_v = (int)chunks.size();
     std::vector<double *> ptrs;
     for (int b = 0; b < nb; b++) {
       for (int q = 0; q < NTAU; q++) ptrs.push_back(h->b[b].tau[q]);
@@ -791,10 +832,22 @@ int setup_exchange(mgpu_handle *h) {
       if (artv)
         for (int q = 0; q < 3; q++) ptrs.push_back(h->b[b].sr[q]);
     }
-    double **dp = nullptr;
-    if ((rc = upload(h, ptrs, &dp))) return rc;
-    h->xv = IfaceArgs{dt, dc, dp, nv};
+    o_v = img.add(ptrs);
   }
+  HIPCK(h, hipMalloc(&h->xtables, img.bytes.size()));
+  HIPCK(h, hipMemcpy(h->xtables, img.bytes.data(), img.bytes.size(), hipMemcpyHostToDevice));
+  char *const at = (char *)h->xtables;
+  for (int s = 0; s < 3; s++)
+    h->xs[s] = IfaceArgs{(FaceTask *)(at + o_st), (IfaceChunk *)(at + o_sc), (double **)(at + o_s[s]), 5};
+  h->xi_tasks = (FaceTask *)(at + o_it);
+  h->xi_chunks = (IfaceChunk *)(at + o_ic);
+  if (h->mixed)
+    for (int s = 0; s < 2; s++) h->xf[s] = IfaceArgs32{h->xi_tasks, h->xi_chunks, (float **)(at + o_f[s]), 5};
+  if (h->c.iorder_visc)
+    h->xv = IfaceArgs{(FaceTask *)(at + o_vt), (IfaceChunk *)(at + o_vc), (double **)(at + o_v), nv};
+  h->nchunks_s = ns;
+  h->nchunks_i = ni;
+  h->nchunks_v = n_v;
   h->exchange_ready = true;
   return 0;
 }
@@ -859,6 +912,9 @@ void stage_plan(const mgpu_handle *h, int v, int &shape, int &kc) {
   }
   double best = 1e30;
   for (int sh : {2, 4, 1, 3}) {
+    // 3-D curvilinear blocks: 64x8 was within 3 % of the fastest at every
+    // size, and keeps one rounding of the halo cells (flux_c3)
+    if (h->c.curvilinear == MGPU_GEOM_C3 && sh != 2) continue;
     double t;
     const int k = plan_kchunk(h, stage_cost(sh), &t);
     if (t < best) {
@@ -1060,6 +1116,7 @@ FilterArgs filter_args(const mgpu_handle *h, const BlockData &bd, int in, int ou
 // changed the tiles).  The stream is idle when they are rewritten.
 int build_tables(mgpu_handle *h) {
   if (h->tables_ready) return 0;
+  set_wrap(h);
   const int nb = (int)h->b.size(), nrk = h->c.nrk;
   const mgpu_case &c = h->c;
   int rc;
@@ -1350,8 +1407,8 @@ int enqueue_step(mgpu_handle *h, int s0) {
     }
     if (h->mixed && !last) {
       ProfScope ps(h, MGPU_K_HALO);
-      HIPCK(h, launch_iface(h->xf[fset_of(irk)], h->nchunks_s, h->stream));
-    } else if ((rc = exchange_state(h, out))) {
+      HIPCK(h, launch_iface(h->xf[fset_of(irk)], h->nchunks_i, h->stream));
+    } else if ((rc = exchange_inner(h, out))) {
       return rc;
     }
     if (h->wall) {
@@ -1393,7 +1450,7 @@ int enqueue_step(mgpu_handle *h, int s0) {
           HIPCK(h, launch_inlet_kf(bd.g, after, before, bd.kf, h->stream));
         }
     }
-    if ((rc = exchange_state(h, s0))) return rc;
+    if ((rc = exchange_inner(h, s0))) return rc;
     if (h->wall) {
       ProfScope ps(h, MGPU_K_HALO);
       if ((rc = enqueue_walls(h, -1, s0))) return rc;
@@ -1836,6 +1893,8 @@ int step(mgpu_handle *h, int nsteps) {
     if (rc) return rc;
     h->cur = next_set(h->c, h->cur);
   }
+  // the ghosts that the steps themselves did not need
+  if (nsteps > 0 && h->nchunks_i != h->nchunks_s) return exchange_state(h, h->cur);
   return 0;
 }
 

@@ -89,8 +89,11 @@ struct mgpu_handle {
   mgpu::IfaceArgs xs[3] = {};  // state set s
   mgpu::IfaceArgs xv = {};     // tau (+ prs, sens)
   mgpu::IfaceArgs32 xf[2] = {};  // mixed precision: FP32 stage sets
-  int nchunks_s = 0, nchunks_v = 0;
-  std::vector<void *> xtables;  // device memory of the exchange tables
+  // the state exchange inside a step (xi), the whole one (nchunks_s) at its end
+  mgpu::FaceTask *xi_tasks = nullptr;
+  mgpu::IfaceChunk *xi_chunks = nullptr;
+  int nchunks_s = 0, nchunks_i = 0, nchunks_v = 0;
+  void *xtables = nullptr;  // device memory of the exchange tables
   bool exchange_ready = false;
   bool ghosts_dirty = false;
   // stage kernel launch parameters: [0] Euler stages, [1] last stage with the

@@ -61,6 +61,11 @@ struct Geom {
   // increment with the one-sided a02 / a20 derivative across the wall; bits
   // as jwall (jadv) and iwall (iadv)
   int iadv, jadv;
+  // axes (bit 0 i, 1 j, 2 k) whose two faces join each other, on a case
+  // whose kernels then read the state and the viscous fluxes beyond them at
+  // the periodic image (lin_w, wrap_k) instead of in ghosts that an exchange
+  // would have to fill after every stage
+  int wrap;
   long n;     // total padded points
 };
 
@@ -84,6 +89,17 @@ __host__ __device__ inline long slab_size(const Geom &g, int axis) {
 
 __host__ __device__ inline idx_t lin(const Geom &g, int i, int j, int k) {
   return (idx_t)(i + G - 1) + (idx_t)g.sx * (idx_t)(j + G - 1) + g.sy * (idx_t)(k + G - 1);
+}
+
+// Row r of an axis of n rows, or its periodic image (on: the axis wraps; r
+// lies at most n rows outside).
+__host__ __device__ inline int wrap_row(int on, int n, int r) {
+  return on ? (r < 1 ? r + n : (r > n ? r - n : r)) : r;
+}
+__host__ __device__ inline int wrap_k(const Geom &g, int k) { return wrap_row(g.wrap & 4, g.nz, k); }
+// Offset of column (i, j) in plane k = 0, at its periodic image where i or j wraps.
+__host__ __device__ inline idx_t lin_w(const Geom &g, int i, int j) {
+  return lin(g, wrap_row(g.wrap & 1, g.nx, i), wrap_row(g.wrap & 2, g.ny, j), 0);
 }
 
 // Load/store at element offset i through a 32-bit byte offset.  The array
