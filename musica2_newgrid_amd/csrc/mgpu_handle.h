@@ -16,7 +16,10 @@ using namespace mgpu;
 struct BlockData {
   Geom g{};
   mgpu_case p{};          // scalars of this block's case (time step, gas, filter amplitudes)
-  double *st[3][5] = {};  // three state sets: st[cur] = U^n, the others stage buffers
+  // three state sets: st[cur] = U^n, the others stage buffers; the arrays of a
+  // set lie st_stride doubles apart in one allocation
+  double *st[3][5] = {};
+  size_t st_stride = 0;
   float *sf[2][5] = {};   // mixed precision: intermediate stage states, FP32 differences with ref
   double *idx[6] = {};    // Cartesian metrics idx,idy,idz,idx_v,idy_v,idz_v
   double *m[10] = {};
@@ -134,6 +137,9 @@ struct mgpu_handle {
   long diag_cap = 0;
   double *cfl_buf = nullptr;   // per-workgroup maxima of mgpu_max_cfl
   long cfl_cap = 0;
+  char *pin = nullptr;         // pinned staging of mgpu_get_state
+  size_t pin_bytes = 0;
+  hipEvent_t pin_ev[8] = {};
 };
 
 namespace mgpu_host {
