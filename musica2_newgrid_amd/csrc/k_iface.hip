@@ -42,7 +42,28 @@ __global__ __launch_bounds__(kIfaceThreads) void k_iface(IfaceArgsT<T> a) {
   for (int v = 0; v < a.nvar; v++) stg(dst[v], pd, ldg(src[t.vmap[v]], ps));
 }
 
+// One thread per value of the caller's rows.
+template <class T>
+__global__ __launch_bounds__(kIfaceThreads) void k_rows(Geom g, const double *__restrict__ src, T *__restrict__ dst,
+                                                        idx_t n) {
+  const idx_t e = (idx_t)blockIdx.x * kIfaceThreads + threadIdx.x;
+  if (e >= n) return;
+  const idx_t w = (idx_t)(g.nx + 2 * G);
+  stg(dst, e / w * (idx_t)g.sx + e % w, (T)ldg(src, e));
+}
+
+template <class T>
+hipError_t rows(const Geom &g, const double *src, T *dst, hipStream_t s) {
+  const idx_t n = (idx_t)host_points(g);
+  hipLaunchKernelGGL(k_rows<T>, dim3((n + kIfaceThreads - 1) / kIfaceThreads), dim3(kIfaceThreads), 0, s, g, src, dst,
+                     n);
+  return hipGetLastError();
+}
+
 }  // namespace
+
+hipError_t launch_rows(const Geom &g, const double *src, double *dst, hipStream_t s) { return rows(g, src, dst, s); }
+hipError_t launch_rows(const Geom &g, const double *src, float *dst, hipStream_t s) { return rows(g, src, dst, s); }
 
 hipError_t launch_iface(const IfaceArgs &a, int nchunks, hipStream_t s) {
   if (nchunks <= 0) return hipSuccess;

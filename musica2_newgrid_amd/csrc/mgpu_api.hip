@@ -948,31 +948,38 @@ struct TuneKey {
 std::mutex g_tune_mu;
 std::map<TuneKey, std::pair<int, int>> g_tune_cache;
 
+// Padded arrays: element 0 lies kLead elements into the allocation.
+template <class T>
+void free_rows(T *&p) {
+  if (p) (void)hipFree(p - kLead);
+  p = nullptr;
+}
+
 void free_block(BlockData &bd) {
   for (auto &s : bd.st) {
-    if (s[0]) (void)hipFree(s[0]);  // the five arrays of a set are one allocation
+    free_rows(s[0]);  // the five arrays of a set are one allocation
     for (auto &p : s) p = nullptr;
   }
   for (auto &s : bd.sf)
-    for (auto &p : s) { if (p) (void)hipFree(p); p = nullptr; }
+    for (auto &p : s) free_rows(p);
   for (auto &p : bd.idx) { if (p) (void)hipFree(p); p = nullptr; }
-  for (auto &p : bd.m) { if (p) (void)hipFree(p); p = nullptr; }
-  for (auto &p : bd.m32) { if (p) (void)hipFree(p); p = nullptr; }
-  for (auto &p : bd.mv) { if (p) (void)hipFree(p); p = nullptr; }
-  for (auto &p : bd.m2) { if (p) (void)hipFree(p); p = nullptr; }
-  for (auto &p : bd.m2v) { if (p) (void)hipFree(p); p = nullptr; }
-  for (auto &p : bd.tau) { if (p) (void)hipFree(p); p = nullptr; }
-  for (auto &p : bd.kv) { if (p) (void)hipFree(p); p = nullptr; }
-  if (bd.prs) (void)hipFree(bd.prs);
-  if (bd.sens) (void)hipFree(bd.sens);
+  for (auto &p : bd.m) free_rows(p);
+  for (auto &p : bd.m32) free_rows(p);
+  for (auto &p : bd.mv) free_rows(p);
+  for (auto &p : bd.m2) free_rows(p);
+  for (auto &p : bd.m2v) free_rows(p);
+  for (auto &p : bd.tau) free_rows(p);
+  for (auto &p : bd.kv) free_rows(p);
+  for (auto &p : bd.sr) free_rows(p);
+  free_rows(bd.prs);
+  free_rows(bd.sens);
   if (bd.wstash) (void)hipFree(bd.wstash);
-  bd.prs = bd.sens = bd.wstash = nullptr;
+  bd.wstash = nullptr;
   for (double **q : {&bd.kimax, &bd.kjmax, &bd.cst, &bd.uin, &bd.ppre, &bd.kf, &bd.wc3[0], &bd.wc3[1], &bd.wt3[0],
                      &bd.wt3[1]}) {
     if (*q) (void)hipFree(*q);
     *q = nullptr;
   }
-  for (auto &p : bd.sr) { if (p) (void)hipFree(p); p = nullptr; }
 }
 
 int dalloc(mgpu_handle *h, double **p, size_t count) {
@@ -986,13 +993,16 @@ int dalloc(mgpu_handle *h, double **p, size_t count) {
   return 0;
 }
 
-int dalloc32(mgpu_handle *h, float **p, size_t count) {
-  hipError_t e = hipMalloc((void **)p, count * sizeof(float));
-  if (e != hipSuccess) {
-    *p = nullptr;
-    return fail(h, MGPU_ENOMEM, "hipMalloc of %zu floats failed: %s", count, hipGetErrorString(e));
-  }
-  e = hipMemset(*p, 0, count * sizeof(float));
+// A padded array (kLead elements before element 0).
+template <class T>
+int dalloc_rows(mgpu_handle *h, T **p, size_t count) {
+  *p = nullptr;
+  T *q = nullptr;
+  const size_t bytes = (count + kRowAlign) * sizeof(T);
+  hipError_t e = hipMalloc((void **)&q, bytes);
+  if (e != hipSuccess) return fail(h, MGPU_ENOMEM, "hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
+  *p = q + kLead;
+  e = hipMemset(q, 0, bytes);
   if (e != hipSuccess) return fail(h, MGPU_EDEVICE, "hipMemset failed: %s", hipGetErrorString(e));
   return 0;
 }
@@ -1567,8 +1577,9 @@ int handle_new(const mgpu_case &c, mgpu_handle **out) {
   return 0;
 }
 
-size_t block_bytes(const mgpu_case &c, int nx, int ny, int nz) {
-  const size_t n = (size_t)(nx + 2 * G) * (ny + 2 * G) * (nz + 2 * G);
+size_t block_bytes(const mgpu_case &c, int nx, int ny, int nz, bool device) {
+  const size_t row = device ? row_length(nx) : nx + 2 * G;
+  const size_t n = row * (ny + 2 * G) * (nz + 2 * G);
   size_t arrays = 15;  // three state sets
   if (c.curvilinear == MGPU_GEOM_C3) arrays += c.iorder_visc ? 20 : 10;
   if (c.iorder_visc)
@@ -1577,7 +1588,7 @@ size_t block_bytes(const mgpu_case &c, int nx, int ny, int nz) {
   if (c.precision == MGPU_PREC_MIXED) bytes += 10 * n * sizeof(float);
   if (c.precision == MGPU_PREC_MIXED && c.curvilinear == MGPU_GEOM_C3) bytes += 9 * n * sizeof(float);
   if (c.curvilinear != MGPU_GEOM_C3) bytes += 6 * (size_t)(nx + ny + nz + 6 * G) * sizeof(double);
-  if (c.curvilinear == MGPU_GEOM_C2) bytes += 10 * (size_t)(nx + 2 * G) * (ny + 2 * G) * sizeof(double);
+  if (c.curvilinear == MGPU_GEOM_C2) bytes += 10 * row * (ny + 2 * G) * sizeof(double);
   return bytes;  // (+ 4*nx*nz doubles of wall state for a block with walls)
 }
 
@@ -1596,7 +1607,7 @@ int handle_add_block(mgpu_handle *h, const mgpu_block &bl, const mgpu_case &p) {
   bd.g.nx = bl.nx;
   bd.g.ny = bl.ny;
   bd.g.nz = bl.nz;
-  bd.g.sx = bl.nx + 2 * G;
+  bd.g.sx = row_length(bl.nx);
   bd.g.sy = (idx_t)bd.g.sx * (idx_t)(bl.ny + 2 * G);
   bd.g.n = (long)bd.g.sy * (bl.nz + 2 * G);
   bd.g.jwall = (is_wall(bl.face_kind[2]) ? 1 : 0) | (is_wall(bl.face_kind[3]) ? 2 : 0);
@@ -1607,31 +1618,31 @@ int handle_add_block(mgpu_handle *h, const mgpu_block &bl, const mgpu_case &p) {
   bd.islip = (is_slip(p, bl.face_kind[0]) ? 1 : 0) | (is_slip(p, bl.face_kind[1]) ? 2 : 0);
   bd.g.ibnd = (is_bound(bl.face_kind[0]) ? 1 : 0) | (is_bound(bl.face_kind[1]) ? 2 : 0);
   bd.g.jbnd = (is_bound(bl.face_kind[2]) ? 1 : 0) | (is_bound(bl.face_kind[3]) ? 2 : 0);
-  bd.bytes = block_bytes(c, bl.nx, bl.ny, bl.nz);
+  bd.bytes = block_bytes(c, bl.nx, bl.ny, bl.nz, true);
   const size_t n = (size_t)bd.g.n;
   int rc = 0;
   bd.st_stride = (n + 31) / 32 * 32;
   for (int s = 0; s < 3 && !rc; s++) {
-    rc = dalloc(h, &bd.st[s][0], 5 * bd.st_stride);
+    rc = dalloc_rows(h, &bd.st[s][0], 5 * bd.st_stride);
     for (int v = 1; v < 5 && !rc; v++) bd.st[s][v] = bd.st[s][0] + v * bd.st_stride;
   }
   if (h->mixed)
     for (int s = 0; s < 2 && !rc; s++)
-      for (int v = 0; v < 5 && !rc; v++) rc = dalloc32(h, &bd.sf[s][v], n);
+      for (int v = 0; v < 5 && !rc; v++) rc = dalloc_rows(h, &bd.sf[s][v], n);
   if (c.curvilinear == MGPU_GEOM_C3) {
-    for (int q = 0; q < 10 && !rc; q++) rc = dalloc(h, &bd.m[q], n);
+    for (int q = 0; q < 10 && !rc; q++) rc = dalloc_rows(h, &bd.m[q], n);
     if (h->mixed)
-      for (int q = 0; q < 9 && !rc; q++) rc = dalloc32(h, &bd.m32[q], n);
+      for (int q = 0; q < 9 && !rc; q++) rc = dalloc_rows(h, &bd.m32[q], n);
     if (c.iorder_visc)
-      for (int q = 0; q < 10 && !rc; q++) rc = dalloc(h, &bd.mv[q], n);
+      for (int q = 0; q < 10 && !rc; q++) rc = dalloc_rows(h, &bd.mv[q], n);
   } else {
     // Cartesian metrics; a 2.5-D block uses idz, idz_v of them and 2-D arrays
     const int len[3] = {bl.nx + 2 * G, bl.ny + 2 * G, bl.nz + 2 * G};
     for (int q = 0; q < 6 && !rc; q++) rc = dalloc(h, &bd.idx[q], (size_t)len[q % 3]);
     if (c.curvilinear == MGPU_GEOM_C2) {
       const size_t n2 = (size_t)bd.g.sx * (bl.ny + 2 * G);
-      for (int q = 0; q < 5 && !rc; q++) rc = dalloc(h, &bd.m2[q], n2);
-      for (int q = 0; q < 5 && !rc; q++) rc = dalloc(h, &bd.m2v[q], n2);
+      for (int q = 0; q < 5 && !rc; q++) rc = dalloc_rows(h, &bd.m2[q], n2);
+      for (int q = 0; q < 5 && !rc; q++) rc = dalloc_rows(h, &bd.m2v[q], n2);
     }
   }
   if ((bd.g.jwall || bd.g.iwall) && !rc)
@@ -1656,14 +1667,14 @@ int handle_add_block(mgpu_handle *h, const mgpu_block &bl, const mgpu_case &p) {
     }
   }
   if (c.iorder_visc) {
-    for (int q = 0; q < NTAU && !rc; q++) rc = dalloc(h, &bd.tau[q], n);
-    for (int q = 0; q < 4 && !rc; q++) rc = dalloc(h, &bd.kv[q], n);
+    for (int q = 0; q < NTAU && !rc; q++) rc = dalloc_rows(h, &bd.tau[q], n);
+    for (int q = 0; q < 4 && !rc; q++) rc = dalloc_rows(h, &bd.kv[q], n);
     if (has_sensor(c)) {
-      if (!rc) rc = dalloc(h, &bd.prs, n);
-      if (!rc) rc = dalloc(h, &bd.sens, n);
+      if (!rc) rc = dalloc_rows(h, &bd.prs, n);
+      if (!rc) rc = dalloc_rows(h, &bd.sens, n);
     }
     if (has_sr(c))
-      for (int q = 0; q < 3 && !rc; q++) rc = dalloc(h, &bd.sr[q], n);
+      for (int q = 0; q < 3 && !rc; q++) rc = dalloc_rows(h, &bd.sr[q], n);
   }
   if (rc) {
     free_block(bd);
@@ -1722,17 +1733,32 @@ int put_metrics_cart(mgpu_handle *h, int block, const double *const *src_in) {
   return 0;
 }
 
+// One array of the caller, hp = host_points(bd.g) values, into a padded array
+// (and, f32 not null, its FP32 copy): through a stage buffer, which holds
+// nothing between steps; the stream is idle before and after.
+int upload_rows(mgpu_handle *h, BlockData &bd, const double *src, double *dst, float *f32 = nullptr) {
+  double *const scratch = bd.st[(h->cur + 1) % 3][0];
+  HIPCK(h, hipStreamSynchronize(h->stream));
+  HIPCK(h, hipMemcpy(scratch, src, sizeof(double) * host_points(bd.g), hipMemcpyHostToDevice));
+  HIPCK(h, launch_rows(bd.g, scratch, dst, h->stream));
+  if (f32) HIPCK(h, launch_rows(bd.g, scratch, f32, h->stream));
+  // (zeros again: the corners of a stage set are never written, and a case
+  // without a filter returns its sets in turn)
+  HIPCK(h, hipMemsetAsync(scratch, 0, sizeof(double) * host_points(bd.g), h->stream));
+  HIPCK(h, hipStreamSynchronize(h->stream));
+  return 0;
+}
+
 int put_metrics_c3(mgpu_handle *h, int block, const double *const *m, const double *const *mv) {
   if (block < 0 || block >= (int)h->b.size()) return fail(h, MGPU_EINVAL, "block %d out of range", block);
   if (h->c.curvilinear != MGPU_GEOM_C3)
     return fail(h, MGPU_ESTATE, "case is not 3-D curvilinear: use mgpu_set_metrics_cart or _c2");
   if (!m) return fail(h, MGPU_EINVAL, "null metric table");
   BlockData &bd = h->b[block];
-  const size_t bytes = sizeof(double) * (size_t)bd.g.n;
   // a relabeled block (walls on its i- or k-faces): the rows of its stored
   // index axes, each array in the stored axis order; the physical components
   // x, y, z and 1/J keep their places
-  std::vector<double> tmp(bd.perm ? (size_t)bd.g.n : 0);
+  std::vector<double> tmp(bd.perm ? host_points(bd.g) : 0);
   auto stored = [&](const double *const *src, int q) -> const double * {
     const double *a = q < 9 ? src[3 * caller_axis(bd.perm, q / 3) + q % 3] : src[q];
     if (!bd.perm) return a;
@@ -1741,21 +1767,19 @@ int put_metrics_c3(mgpu_handle *h, int block, const double *const *m, const doub
   };
   for (int q = 0; q < 10; q++)
     if (!m[q]) return fail(h, MGPU_EINVAL, "metric %d is null", q);
-  std::vector<float> f(bd.m32[0] ? (size_t)bd.g.n : 0);
+  // (the mixed path's FP32 copies of the flux metric terms are rounded on the device)
   for (int q = 0; q < 10; q++) {
-    const double *a = stored(m, q);
-    HIPCK(h, hipMemcpy(bd.m[q], a, bytes, hipMemcpyHostToDevice));
-    if (bd.m32[0] && q < 9) {
-      // the mixed path's FP32 copies of the flux metric terms
-      for (size_t e = 0; e < f.size(); e++) f[e] = (float)a[e];
-      HIPCK(h, hipMemcpy(bd.m32[q], f.data(), f.size() * sizeof(float), hipMemcpyHostToDevice));
-    }
+    const int rc = upload_rows(h, bd, stored(m, q), bd.m[q], q < 9 ? bd.m32[q] : nullptr);
+    if (rc) return rc;
   }
   if (h->c.iorder_visc) {
     if (!mv) return fail(h, MGPU_EINVAL, "viscous metric table is null");
     for (int q = 0; q < 10; q++)
       if (!mv[q]) return fail(h, MGPU_EINVAL, "viscous metric %d is null", q);
-    for (int q = 0; q < 10; q++) HIPCK(h, hipMemcpy(bd.mv[q], stored(mv, q), bytes, hipMemcpyHostToDevice));
+    for (int q = 0; q < 10; q++) {
+      const int rc = upload_rows(h, bd, stored(mv, q), bd.mv[q]);
+      if (rc) return rc;
+    }
   }
   bd.have_metrics = true;
   return 0;
@@ -1777,7 +1801,8 @@ int put_metrics_c2(mgpu_handle *h, int block, const double *const *m2, const dou
     const int from[5] = {3, 1, 2, 0, 4};
     const double sign[5] = {1.0, -1.0, -1.0, 1.0, 1.0};
     for (int q = 0; q < 5; q++) {
-      for (size_t e = 0; e < n2; e++) row[e] = sign[q] * src[from[q]][e];
+      const size_t w = (size_t)bd.g.nx + 2 * G;
+      for (size_t e = 0; e < w * (bd.g.ny + 2 * G); e++) row[e / w * bd.g.sx + e % w] = sign[q] * src[from[q]][e];
       HIPCK(h, hipMemcpy(dst[q], row.data(), n2 * sizeof(double), hipMemcpyHostToDevice));
     }
     return 0;
@@ -1798,7 +1823,6 @@ int put_metrics_c2(mgpu_handle *h, int block, const double *const *m2, const dou
 int put_state(mgpu_handle *h, int block, const double *const *src_in) {
   if (block < 0 || block >= (int)h->b.size()) return fail(h, MGPU_EINVAL, "block %d out of range", block);
   BlockData &bd = h->b[block];
-  const size_t bytes = sizeof(double) * (size_t)bd.g.n;
   for (int v = 0; v < 5; v++)
     if (!src_in[v]) return fail(h, MGPU_EINVAL, "state array %d is null", v);
   // a relabeled block: the caller's arrays in the stored axis order
@@ -1807,15 +1831,17 @@ int put_state(mgpu_handle *h, int block, const double *const *src_in) {
   for (int v = 0; v < 5; v++) {
     const double *u = src_in[caller_var(bd.vperm, v)];
     if (bd.perm) {
-      tmp[v].resize((size_t)bd.g.n);
+      tmp[v].resize(host_points(bd.g));
       relabel_array(bd.g, bd.perm, u, tmp[v].data(), true);
       u = tmp[v].data();
     }
     sp[v] = u;
   }
   const double *const *src = sp;
-  HIPCK(h, hipStreamSynchronize(h->stream));
-  for (int v = 0; v < 5; v++) HIPCK(h, hipMemcpy(bd.st[h->cur][v], src[v], bytes, hipMemcpyHostToDevice));
+  for (int v = 0; v < 5; v++) {
+    const int rc = upload_rows(h, bd, src[v], bd.st[h->cur][v]);
+    if (rc) return rc;
+  }
   bd.have_state = true;
   h->ghosts_dirty = true;  // the exchange runs before the next use of the ghosts
   bd.bc_start = bd.kimax || bd.kjmax || bd.uin;
@@ -1829,7 +1855,7 @@ int put_state(mgpu_handle *h, int block, const double *const *src_in) {
       double acc = 0.0;
       for (int k = 1; k <= g.nz; k++)
         for (int j = 1; j <= g.ny; j++) {
-          const double *row = src[v] + lin(g, 1, j, k);
+          const double *row = src[v] + G + (size_t)(g.nx + 2 * G) * ((size_t)(j + G - 1) + (size_t)(g.ny + 2 * G) * (k + G - 1));
           for (int i = 0; i < g.nx; i++) acc += row[i];
         }
       mean[v] = acc / ((double)g.nx * g.ny * g.nz);
@@ -1886,16 +1912,21 @@ int stage_reserve(mgpu_handle *h, size_t bytes) {
   return 0;
 }
 
-// The five arrays of a state set (one piece of device memory, `stride`
-// doubles apart) to n doubles each at dst[v], after the work on h->stream.
+// The five arrays of block bd's state set `set` (one piece of device memory)
+// to the caller's arrays dst[v], after the work on h->stream.
 // A copy into pageable memory runs at 10 GB/s here: one thread copies out of
 // the runtime's staging buffer and takes the first-touch faults of a new
 // array.  Through pinned slots, with the faults and the copies out of the
 // slots spread over a few threads, the same 337 MB take 7.9 instead of 33 ms
 // (43 GB/s, the link); a 16^3 state (0.7 MB) is one copy of 21 us instead of
 // five that take 75.
-int fetch_set(mgpu_handle *h, const double *src, size_t stride, size_t n, double *const *dst) {
-  const size_t total = 5 * stride * sizeof(double), sb = stride * sizeof(double), nb = n * sizeof(double);
+int fetch_set(mgpu_handle *h, const BlockData &bd, int set, double *const *dst) {
+  const Geom &g = bd.g;
+  const double *const src = bd.st[set][0];
+  const size_t sb = bd.st_stride * sizeof(double), total = 5 * sb;
+  // rows of the device and of the caller in bytes, rows of an array
+  const size_t dr = (size_t)g.sx * sizeof(double), hr = (size_t)(g.nx + 2 * G) * sizeof(double);
+  const size_t nr = (size_t)(g.ny + 2 * G) * (size_t)(g.nz + 2 * G);
   size_t slot = (total / 16 + 4095) / 4096 * 4096;
   if (total <= kSlotMin * 4) slot = (total + 4095) / 4096 * 4096;
   else if (slot < kSlotMin) slot = kSlotMin;
@@ -1904,14 +1935,19 @@ int fetch_set(mgpu_handle *h, const double *src, size_t stride, size_t n, double
   const int ns = nch < (size_t)kSlots ? (int)nch : kSlots;
   if (stage_reserve(h, slot * ns) != 0) {
     HIPCK(h, hipStreamSynchronize(h->stream));
-    for (int v = 0; v < 5; v++) HIPCK(h, hipMemcpy(dst[v], src + v * stride, nb, hipMemcpyDeviceToHost));
+    for (int v = 0; v < 5; v++)
+      HIPCK(h, hipMemcpy2D(dst[v], hr, bd.st[set][v], dr, hr, nr, hipMemcpyDeviceToHost));
     return 0;
   }
   // bytes [o, o + len) of the set lie at `at` in pinned memory
   auto scatter = [&](size_t o, size_t len, const char *at) {
     for (size_t v = o / sb; v < 5 && v * sb < o + len; v++) {
-      const size_t a = o > v * sb ? o : v * sb, e = o + len < v * sb + nb ? o + len : v * sb + nb;
-      if (a < e) memcpy((char *)dst[v] + (a - v * sb), at + (a - o), e - a);
+      for (size_t r = o > v * sb ? (o - v * sb) / dr : 0; r < nr; r++) {
+        const size_t row = v * sb + r * dr;  // bytes of the row that this piece holds: [a, e)
+        if (row >= o + len) break;
+        const size_t a = o > row ? o : row, e = o + len < row + hr ? o + len : row + hr;
+        if (a < e) memcpy((char *)dst[v] + r * hr + (a - row), at + (a - o), e - a);
+      }
     }
   };
   auto len_of = [&](size_t c) { return c + 1 < nch ? slot : total - c * slot; };
@@ -1982,18 +2018,16 @@ int fetch_set(mgpu_handle *h, const double *src, size_t stride, size_t n, double
 int get_state(mgpu_handle *h, int block, double *const *dst) {
   if (block < 0 || block >= (int)h->b.size()) return fail(h, MGPU_EINVAL, "block %d out of range", block);
   BlockData &bd = h->b[block];
-  const size_t bytes = sizeof(double) * (size_t)bd.g.n;
   for (int v = 0; v < 5; v++)
     if (!dst[v]) return fail(h, MGPU_EINVAL, "state array %d is null", v);
   int rc = refresh_ghosts(h);
   if (rc) return rc;
-  if (!bd.perm) return fetch_set(h, bd.st[h->cur][0], bd.st_stride, (size_t)bd.g.n, dst);
-  HIPCK(h, hipStreamSynchronize(h->stream));
-  std::vector<double> tmp((size_t)bd.g.n);
-  for (int v = 0; v < 5; v++) {
-    HIPCK(h, hipMemcpy(tmp.data(), bd.st[h->cur][v], bytes, hipMemcpyDeviceToHost));
-    relabel_array(bd.g, bd.perm, tmp.data(), dst[caller_var(bd.vperm, v)], false);
-  }
+  if (!bd.perm) return fetch_set(h, bd, h->cur, dst);
+  const size_t hp = host_points(bd.g);
+  std::vector<double> tmp(5 * hp);
+  double *const t[5] = {&tmp[0], &tmp[hp], &tmp[2 * hp], &tmp[3 * hp], &tmp[4 * hp]};
+  if ((rc = fetch_set(h, bd, h->cur, t))) return rc;
+  for (int v = 0; v < 5; v++) relabel_array(bd.g, bd.perm, t[v], dst[caller_var(bd.vperm, v)], false);
   return 0;
 }
 

@@ -158,8 +158,9 @@ int handle_new(const mgpu_case &c, mgpu_handle **out);
 int handle_add_block(mgpu_handle *h, const mgpu_block &bl, const mgpu_case &p);
 // Frees block i and removes it from the handle (the other blocks keep their order).
 int handle_remove_block(mgpu_handle *h, int i);
-// Device bytes a block of extents nx,ny,nz needs under the flags of c.
-size_t block_bytes(const mgpu_case &c, int nx, int ny, int nz);
+// Bytes of the arrays a block of extents nx,ny,nz needs under the flags of c:
+// with rows of nx + 2G values, or (device) as long as they are on the device.
+size_t block_bytes(const mgpu_case &c, int nx, int ny, int nz, bool device);
 // Uploads metrics / state of block i (host arrays in the padded layout).
 int put_metrics_cart(mgpu_handle *h, int i, const double *const *a6);
 int put_metrics_c3(mgpu_handle *h, int i, const double *const *m, const double *const *mv);

@@ -176,8 +176,10 @@ int mgpu_server_submit(mgpu_server *s, const mgpu_case *c, const double *const *
   r->blk = bl;
   r->nsteps = nsteps;
   r->n = n;
-  r->dev_bytes = block_bytes(*c, bl.nx, bl.ny, bl.nz);
-  if ((int64_t)r->dev_bytes > s->budget) return sfail(s, MGPU_EINVAL, "request larger than the whole budget");
+  r->dev_bytes = block_bytes(*c, bl.nx, bl.ny, bl.nz, true);
+  // refused by the size of the caller's arrays; one that fits so is admitted
+  // alone even where its device rows are longer
+  if ((int64_t)block_bytes(*c, bl.nx, bl.ny, bl.nz, false) > s->budget) return sfail(s, MGPU_EINVAL, "request larger than the whole budget");
   if (c->curvilinear == MGPU_GEOM_C2) {
     const size_t n2 = (size_t)(bl.nx + 2 * G) * (bl.ny + 2 * G), nz = (size_t)bl.nz + 2 * G;
     const bool visc = c->iorder_visc != 0;
@@ -231,7 +233,7 @@ int mgpu_server_tick(mgpu_server *s, int max_steps, int *n_resident, int *n_queu
   // admit in submission order while the budget allows
   while (!s->queue.empty()) {
     Request *r = s->queue.front();
-    if (s->used + (int64_t)r->dev_bytes > s->budget) break;
+    if (s->used && s->used + (int64_t)r->dev_bytes > s->budget) break;
     if ((rc = admit(s, r))) return rc;
     s->queue.erase(s->queue.begin());
   }
