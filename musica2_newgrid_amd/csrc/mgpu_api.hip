@@ -927,6 +927,22 @@ void stage_plan(const mgpu_handle *h, int v, int &shape, int &kc) {
   }
 }
 
+// The viscous terms in one kernel (k_viscdiv): every axis of every block
+// wraps, no spectral radii are wanted with them, and the chunks are long
+// enough for its four planes of warm-up.  Against k_visc and k_vdiv one after
+// the other, medians of one run: 16^3 (chunks of 1 plane) 16 us against 12,
+// 64^3 (2) 24 against 22, 113x75x51 (5) 38 against 41, 161x97x65 c3 (11) 100
+// against 123, 192^3 292 against 415, 256x128x96 c3 206 against 294,
+// 512x256x128 2.5-D 592 against 1118.  Not in mixed precision: the last bits
+// of K_v differ from the two kernels', which FP64 stages carry on as 1e-13 of
+// the state, but FP32 flux arithmetic turned into 1.9e-7 of it.
+bool fused_visc(const mgpu_handle *h) {
+  if (!h->c.iorder_visc || has_sr(h->c) || h->mixed) return false;
+  for (const auto &bd : h->b)
+    if (bd.g.wrap != 7) return false;
+  return plan_kchunk(h, MarchCost{32, 16, kCUs, 1.0, 1.0}, nullptr) >= 5;
+}
+
 // k-chunk of k_visc (kind 0), k_vdiv (1) and the filter (2), all 32x16 tiles
 // of 512 threads: one workgroup per CU at their register counts, but two of
 // k_vdiv on Cartesian and 2.5-D blocks (120 VGPRs).
@@ -1155,6 +1171,7 @@ int build_tables(mgpu_handle *h) {
     h->nt_stage[v] = stage_ranges(h, v, tr[v]);
     stage_plan(h, v, h->run_shape[v], kc);
   }
+  h->visc_fused = fused_visc(h);
   const int kcv = aux_kchunk(h, 0), kcd = aux_kchunk(h, 1), kcf = aux_kchunk(h, 2);
   std::vector<Batch<StageArgs>> st((size_t)3 * nrk * nb);
   std::vector<Batch<ViscArgs>> vi(3 * nb);
@@ -1191,6 +1208,7 @@ int build_tables(mgpu_handle *h) {
       for (int v = 0; v < 5; v++) va.u0.v[v] = bd.st[s0][v];
       va.met = metrics_of(bd);
       for (int q = 0; q < NTAU; q++) va.tau[q] = bd.tau[q];
+      for (int q = 0; q < 4; q++) va.kv[q] = bd.kv[q];
       va.prs = bd.prs;
       va.sens = bd.sens;
       for (int q = 0; q < 3; q++) va.sr[q] = bd.sr[q];
@@ -1388,7 +1406,10 @@ int enqueue_step(mgpu_handle *h, int s0) {
   for (int irk = 1; irk <= nrk; irk++) {
     const bool last = irk == nrk;
     const int out = (irk % 2 == 1) ? sa : sb;
-    if (last && visc) {
+    if (last && visc && h->visc_fused) {
+      ProfScope ps(h, MGPU_K_VISC);
+      HIPCK(h, launch_viscdiv(h->d_visc + s0 * nb, nb, h->nt_visc, geo, h->stream));
+    } else if (last && visc) {
       ProfScope ps(h, MGPU_K_VISC);
       HIPCK(h, launch_visc(h->d_visc + s0 * nb, nb, h->nt_visc, geo, h->stream));
       if (h->bnd)
@@ -2219,10 +2240,13 @@ int tune_aux(mgpu_handle *h, bool force, hipEvent_t e0, hipEvent_t e1) {
   for (const auto &bd : h->b) maxnz = bd.g.nz > maxnz ? bd.g.nz : maxnz;
   const int kcs[] = {0, 4, 8, 16, 32, 64, 128, 256};
   int rc = 0;
+  h->visc_fused = fused_visc(h);
   for (int kind = 0; kind < 3 && !rc; kind++) {
     if (kind < 2 && !h->c.iorder_visc) continue;
+    if (kind == 1 && h->visc_fused) continue;
     if (kind == 2 && h->c.filter == MGPU_FILTER_NONE) continue;
-    TuneKey key{h->device, h->c.curvilinear, 10 + 3 * h->c.filter + kind + (h->mixed ? 100 : 0), {}};
+    const int what = kind + (h->mixed ? 100 : 0) + (kind == 0 && h->visc_fused ? 200 : 0);
+    TuneKey key{h->device, h->c.curvilinear, 10 + 3 * h->c.filter + what, {}};
     for (const auto &bd : h->b) key.dims.insert(key.dims.end(), {bd.g.nx, bd.g.ny, bd.g.nz});
     if (!force) {
       std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -2256,6 +2280,7 @@ int tune_aux(mgpu_handle *h, bool force, hipEvent_t e0, hipEvent_t e1) {
         HIPCK(h, hipMemcpy(h->d_tune_f, tab.data(), nb * sizeof(tab[0]), hipMemcpyHostToDevice));
       }
       auto launch = [&]() -> hipError_t {
+        if (kind == 0 && h->visc_fused) return launch_viscdiv(h->d_visc + s0 * nb, nb, h->nt_visc, geo, h->stream);
         if (kind == 0) return launch_visc(h->d_visc + s0 * nb, nb, h->nt_visc, geo, h->stream);
         if (kind == 1) return launch_vdiv(h->d_vdiv, nb, h->nt_vdiv, geo, h->stream);
         if (h->c.filter == MGPU_FILTER_SF)

@@ -110,6 +110,7 @@ struct mgpu_handle {
   int kchunk[2] = {0, 0};
   // planes per workgroup of k_visc, k_vdiv and the filter (0: chosen by size)
   int kc_aux[3] = {0, 0, 0};
+  bool visc_fused = false;  // the viscous terms by k_viscdiv (set with the launch tables)
   // tile numbering (TileRange::jfirst) of the stage variants and of k_visc,
   // k_vdiv and the filter
   int jfirst[2] = {0, 0};

@@ -304,7 +304,8 @@ struct ViscArgs {
   Gas gas;
   CState u0;          // U^n
   Metrics met;
-  double *tau[NTAU];  // out: interior points
+  double *tau[NTAU];  // out: interior points (k_visc)
+  double *kv[4];      // out: the viscous increment (k_viscdiv)
   double *prs;        // out: p(U^n), interior points (shock filter)
   double *sens;       // out: Ducros sensor, interior points (shock filter)
   double *sr[3];      // out: |u|+c, |v|+c, |w|+c of U^n, interior points (artificial viscosity,
@@ -498,6 +499,8 @@ hipError_t launch_stage(const Batch<StageArgs> *tab, int nb, int ntiles, int geo
                         int mode, int wall, hipStream_t s);
 TileRange visc_tiles(const Geom &g, int kchunk);
 hipError_t launch_visc(const Batch<ViscArgs> *tab, int nb, int ntiles, int geo, hipStream_t s);
+// k_visc and k_vdiv in one, for batches of blocks whose three axes wrap
+hipError_t launch_viscdiv(const Batch<ViscArgs> *tab, int nb, int ntiles, int geo, hipStream_t s);
 TileRange vdiv_tiles(const Geom &g, int kchunk);
 hipError_t launch_vdiv(const Batch<VdivArgs> *tab, int nb, int ntiles, int geo, hipStream_t s);
 TileRange filter_tiles(const Geom &g, int kchunk);
