@@ -18,10 +18,11 @@
 //
 // 2.5-D layout: the state of the tile + 5-cell halos of the current k plane
 // sits in LDS for the i/j stencils, the own column keeps an 11-deep register
-// queue for k.  The shock filter also stages p(U^n) and the Ducros sensor
-// and computes each pressure sensor once per plane in LDS.  Halo cells are
-// statically assigned to lanes so that all global loads of a plane are
-// issued in one batch.
+// queue for k.  The shock filter also stages p(U^n) and computes each
+// pressure sensor once per plane in LDS.  Halo cells are statically assigned
+// to lanes so that all global loads of a plane are issued in one batch.
+// k_shock is the shock filter alone; k_filter_shock takes it with the Edoh
+// switch, and the artificial viscosities.
 #include <type_traits>
 
 #include "mgpu_internal.h"
@@ -121,12 +122,23 @@ __device__ __forceinline__ R fwall(const R *y, int s, int hw, double chi) {
   }
 }
 
+// A plane of the tile and its 5-cell halos in LDS: a cross of rows (j0-5..)
+// and columns (i0-5..) whose corners are neither written nor read; every cell
+// of the tile once, for the i- and the j-stencils alike.
+constexpr int SW = FX + 10, SH = FY + 10;
+static_assert(NS == 1, "one halo cell per lane");
+
+// k_filter_sf and k_shock march along k with one barrier per plane: while the
+// stencils of plane k run from one LDS buffer, plane k+1 is written to the
+// other and the loads of plane k+2 are in flight.  One workgroup of 8 waves
+// per CU (its register queue), so nothing else hides what a wave waits for.
+// k_filter_sf, against two barriers and the plane staged twice: 192^3 268 us,
+// now 239 (its 10 words per cell take 113 us), 384x192x96 with walls 292,
+// now 273.
 template <bool WALL>
 __global__ __launch_bounds__(FT, 2) void k_filter_sf(const Batch<FilterArgs> *__restrict__ tab, int nb, int ntiles) {
-
   using R = double;
-  __shared__ R sux[5][FY][FX + 10];
-  __shared__ R suy[5][FY + 10][FX];
+  __shared__ R su[2][5][SH][SW];
   int i0, j0, kbeg, kend;
   const FilterArgs &a = tile_of(tab, nb, ntiles, i0, j0, kbeg, kend);
   // the block's array pointers, read once from the table into registers
@@ -136,70 +148,72 @@ __global__ __launch_bounds__(FT, 2) void k_filter_sf(const Batch<FilterArgs> *__
   const int tx = threadIdx.x % FX, ty = threadIdx.x / FX;
   const int i = i0 + tx, j = j0 + ty;
   const bool own = i <= g.nx && j <= g.ny;
-  const bool needx = i <= g.nx + 5 && j <= g.ny, needy = i <= g.nx && j <= g.ny + 5;
+  // points past the end of a partial tile that its stencils reach
+  const bool past = !own && ((i <= g.nx + 5 && j <= g.ny) || (i <= g.nx && j <= g.ny + 5));
   const idx_t sz = g.sy, own_off = lin_w(g, i, j);
   Halo hl;
   halo_setup(g, i0, j0, hl);
+  const int hr = hl.xdir[0] ? hl.r[0] + 5 : hl.r[0], hc = hl.xdir[0] ? hl.c[0] : hl.c[0] + 5;
+  const int hw = WALL ? jhalf(g, j) : 5;
+  const int hwi = WALL ? ihalf(g, i) : 5;
   R dd[6];
 #pragma unroll
   for (int l = 0; l < 6; l++) dd[l] = (R)a.dd[l];
 
-  R q[11][5];
+  // own column: planes k-5..k+5, plane k+6 in flight; a point past the end
+  // has its plane k+1 there instead
+  R q[11][5], qn[5], uh[5];
   if (own) {
 #pragma unroll
     for (int l = 0; l < 10; l++) ldr(uinp, own_off + (idx_t)wrap_k(g, kbeg - 5 + l) * sz, q[l]);
   }
-  // the state loads of a plane (queue point k+5, pencil cell, halo cells)
-  // are issued one plane ahead, during the previous plane's stencils
-  R qn[5], uc[5], uh[NS][5];
-  {
-    const idx_t pk = own_off + (idx_t)kbeg * sz;
-    if (own) ldr(uinp, own_off + (idx_t)wrap_k(g, kbeg + 5) * sz, qn);
-    if (!own && (needx || needy)) ldr(uinp, pk, uc);
+  if (past) ldr(uinp, own_off + (idx_t)kbeg * sz, qn);
+  if (hl.on[0]) ldr(uinp, hl.off[0] + (idx_t)kbeg * sz, uh);
+  auto stage = [&](int b, const R c[5]) __attribute__((always_inline)) {
+    if (own || past) {
 #pragma unroll
-    for (int s = 0; s < NS; s++)
-      if (hl.on[s]) ldr(uinp, hl.off[s] + (idx_t)kbeg * sz, uh[s]);
+      for (int v = 0; v < 5; v++) su[b][v][ty + 5][tx + 5] = c[v];
+    }
+    if (hl.on[0]) {
+#pragma unroll
+      for (int v = 0; v < 5; v++) su[b][v][hr][hc] = uh[v];
+    }
+  };
+  {
+    R c[5];
+#pragma unroll
+    for (int v = 0; v < 5; v++) c[v] = own ? q[5][v] : qn[v];
+    stage(kbeg & 1, c);
   }
+  if (own) ldr(uinp, own_off + (idx_t)wrap_k(g, kbeg + 5) * sz, qn);
+  if (kbeg < kend) {
+    if (past) ldr(uinp, own_off + (idx_t)(kbeg + 1) * sz, qn);
+    if (hl.on[0]) ldr(uinp, hl.off[0] + (idx_t)(kbeg + 1) * sz, uh);
+  }
+  __syncthreads();
+
   for (int k = kbeg; k <= kend; k++) {
     const idx_t pk = own_off + (idx_t)k * sz;
+    const int b = k & 1;
     if (own) {
 #pragma unroll
       for (int v = 0; v < 5; v++) q[10][v] = qn[v];
     }
-    if (needx || needy) {
-#pragma unroll
-      for (int v = 0; v < 5; v++) {
-        const R x = own ? q[5][v] : uc[v];
-        if (needx) sux[v][ty][tx + 5] = x;
-        if (needy) suy[v][ty + 5][tx] = x;
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-      if (hl.on[s]) {
-#pragma unroll
-        for (int v = 0; v < 5; v++) {
-          if (hl.xdir[s]) sux[v][hl.r[s]][hl.c[s]] = uh[s][v];
-          else suy[v][hl.r[s]][hl.c[s]] = uh[s][v];
-        }
-      }
-    }
-    __syncthreads();
     if (k < kend) {
-      const idx_t pn = pk + sz;
-      if (own) ldr(uinp, own_off + (idx_t)wrap_k(g, k + 6) * sz, qn);
-      if (!own && (needx || needy)) ldr(uinp, pn, uc);
+      R c[5];
 #pragma unroll
-      for (int s = 0; s < NS; s++)
-        if (hl.on[s]) ldr(uinp, hl.off[s] + (idx_t)(k + 1) * sz, uh[s]);
+      for (int v = 0; v < 5; v++) c[v] = own ? q[6][v] : qn[v];
+      stage(b ^ 1, c);
+      if (own) ldr(uinp, own_off + (idx_t)wrap_k(g, k + 6) * sz, qn);
+      if (k + 2 <= kend) {
+        if (past) ldr(uinp, pk + 2 * sz, qn);
+        if (hl.on[0]) ldr(uinp, hl.off[0] + (idx_t)(k + 2) * sz, uh);
+      }
     }
     if (own) {
-      const int hw = WALL ? jhalf(g, j) : 5;
-      const int hwi = WALL ? ihalf(g, i) : 5;
 #pragma unroll
       for (int v = 0; v < 5; v++) {
-        const R *x = &sux[v][ty][tx + 5];
-        const R *y = &suy[v][ty + 5][tx];
+        const R *x = &su[b][v][ty + 5][tx + 5];
         R K;
         if (!WALL || hwi == 5) {
           K = dd[0] * x[0] + dd[1] * (x[1] + x[-1]) + dd[2] * (x[2] + x[-2]) + dd[3] * (x[3] + x[-3]) +
@@ -209,11 +223,11 @@ __global__ __launch_bounds__(FT, 2) void k_filter_sf(const Batch<FilterArgs> *__
           if constexpr (WALL) K = fwall<R>(x, 1, hwi, a.chi);
         }
         if (!WALL || hw == 5) {
-          K = K + dd[0] * y[0] + dd[1] * (y[FX] + y[-FX]) + dd[2] * (y[2 * FX] + y[-2 * FX]) +
-              dd[3] * (y[3 * FX] + y[-3 * FX]) + dd[4] * (y[4 * FX] + y[-4 * FX]) +
-              dd[5] * (y[5 * FX] + y[-5 * FX]);
+          K = K + dd[0] * x[0] + dd[1] * (x[SW] + x[-SW]) + dd[2] * (x[2 * SW] + x[-2 * SW]) +
+              dd[3] * (x[3 * SW] + x[-3 * SW]) + dd[4] * (x[4 * SW] + x[-4 * SW]) +
+              dd[5] * (x[5 * SW] + x[-5 * SW]);
         } else {
-          if constexpr (WALL) K = K + fwall<R>(y, FX, hw, a.chi);
+          if constexpr (WALL) K = K + fwall<R>(x, SW, hw, a.chi);
         }
         K = K + dd[0] * q[5][v] + dd[1] * (q[6][v] + q[4][v]) + dd[2] * (q[7][v] + q[3][v]) +
             dd[3] * (q[8][v] + q[2][v]) + dd[4] * (q[9][v] + q[1][v]) + dd[5] * (q[10][v] + q[0][v]);
@@ -281,6 +295,225 @@ __device__ __forceinline__ double edoh_mul(const FilterArgs &a, int d, idx_t p, 
   return fmin(1.0, cfl / a.chi);
 }
 
+// The shock filter (without the Edoh switch).  Sensors run one plane ahead of
+// the stencils, p two.  Along k the face k+1/2 of a plane is the face k-1/2 of
+// the next and is computed once, as is its pressure sensor.  With three
+// barriers per plane, the plane staged twice (for i and for j) and both k
+// faces of every point: 512x256x128 c3 with walls 876 us, 2.5-D 862 us,
+// 113x75x51 38 us; now 645, 683 and 33 us.  It moves 1.62 GB on the first
+// (320 us at the rate of a large copy): waves wait for 38 % of their cycles
+// and 27 % more for an issue slot, vector instructions take 25 %.
+// WALL: blocks with boundary faces on i or j; rows 1..5 and n-4..n of a
+// bounded axis get no increment along it here (k_shock_wall adds it with the
+// reduced faces of the boundary closure).
+template <bool WALL>
+__global__ __launch_bounds__(FT, 2) void k_shock(const Batch<FilterArgs> *__restrict__ tab, int nb, int ntiles) {
+  using R = double;
+  __shared__ R su[2][5][SH][SW];
+  __shared__ double spr[2][FY + 4][FX + 4];  // p from (i0-2, j0-2)
+  __shared__ double psx[2][FY][FX + 2];      // psens_x at i0-1 .. i0+FX
+  __shared__ double psy[2][FY + 2][FX];      // psens_y at j0-1 .. j0+FY
+
+  int i0, j0, kbeg, kend;
+  const FilterArgs &a = tile_of(tab, nb, ntiles, i0, j0, kbeg, kend);
+  // the block's array pointers, read once from the table into registers
+  const CState uinp = a.uin;
+  const State uoutp = a.uout;
+  const double *const prsp = a.prs, *const sensp = a.sens;
+  const Geom &g = a.g;
+  const int tid = threadIdx.x, tx = tid % FX, ty = tid / FX;
+  const int i = i0 + tx, j = j0 + ty;
+  const bool own = i <= g.nx && j <= g.ny;
+  // points past the end of a partial tile: state, p and sensor that it reads
+  const bool past = !own && ((i <= g.nx + 5 && j <= g.ny) || (i <= g.nx && j <= g.ny + 5));
+  const bool pon = (i <= g.nx + 2 && j <= g.ny) || (i <= g.nx && j <= g.ny + 2);
+  const bool sxon = i <= g.nx + 1 && j <= g.ny, syon = i <= g.nx && j <= g.ny + 1;
+  const bool duc = sensp != nullptr;
+  const double cs = a.csens;
+  const idx_t sz = g.sy, own_off = lin_w(g, i, j);
+  Halo hl;
+  halo_setup(g, i0, j0, hl);
+  const bool hon = hl.on[0], hx = hl.xdir[0];
+  const int hr = hx ? hl.r[0] + 5 : hl.r[0], hc = hx ? hl.c[0] : hl.c[0] + 5;
+  const idx_t h_off = hl.off[0];
+  // halo cells whose p (two rows) and sensor (one row) are needed
+  const int hn = hx ? hc - 5 : hr - 5, hm = hx ? FX : FY;
+  const bool hpon = hon && hn >= -2 && hn <= hm + 1 && (hx ? i0 + hn <= g.nx + 2 : j0 + hn <= g.ny + 2);
+  const bool hson = hon && hn >= -1 && hn <= hm && (hx ? i0 + hn <= g.nx + 1 : j0 + hn <= g.ny + 1);
+
+  R q[11][5], qn[5], uh[5];  // as k_filter_sf
+  double qp[5];              // p at k-2..k+2
+  double qpn = 0.0, ph = 0.0, sc = 1.0, scn = 1.0, sh = 1.0;
+  auto put_u = [&](int b, const R c[5]) __attribute__((always_inline)) {
+    if (own || past) {
+#pragma unroll
+      for (int v = 0; v < 5; v++) su[b][v][ty + 5][tx + 5] = c[v];
+    }
+    if (hon) {
+#pragma unroll
+      for (int v = 0; v < 5; v++) su[b][v][hr][hc] = uh[v];
+    }
+  };
+  auto put_p = [&](int b, double pc) __attribute__((always_inline)) {
+    if (pon) spr[b][ty + 2][tx + 2] = pc;
+    if (hpon) spr[b][hr - 3][hc - 3] = ph;
+  };
+  // pressure sensors of a plane, from sc (own cell) and sh (halo cell)
+  auto sensors = [&](int b) __attribute__((always_inline)) {
+    const double *c = &spr[b][ty + 2][tx + 2];
+    constexpr int W = FX + 4;
+    if (sxon) psx[b][ty][tx + 1] = psens3(c[-1], c[0], c[1], sc, cs);
+    if (syon) psy[b][ty + 1][tx] = psens3(c[-W], c[0], c[W], sc, cs);
+    if (hson) {
+      const double *h = &spr[b][hr - 3][hc - 3];
+      const int d = hx ? 1 : W;
+      const double e = psens3(h[-d], h[0], h[d], sh, cs);
+      if (hx) psx[b][hr - 5][hc - 4] = e;
+      else psy[b][hr - 4][hc - 5] = e;
+    }
+  };
+
+  // ---- planes kbeg (state, p, sensors) and kbeg+1 (p) ----
+  R dlo[5];        // D at the face k-1/2
+  double ps0 = 0;  // pressure sensor along k at k
+#pragma unroll
+  for (int v = 0; v < 5; v++) dlo[v] = R(0);
+  if (own) {
+#pragma unroll
+    for (int l = 0; l < 10; l++) ldr(uinp, own_off + (idx_t)wrap_k(g, kbeg - 5 + l) * sz, q[l]);
+#pragma unroll
+    for (int l = 0; l < 2; l++) qp[l] = ldg(prsp, own_off + (idx_t)wrap_k(g, kbeg - 2 + l) * sz);
+  }
+  if (pon) {
+#pragma unroll
+    for (int l = 2; l < 4; l++) qp[l] = ldg(prsp, own_off + (idx_t)wrap_k(g, kbeg - 2 + l) * sz);
+  }
+  if (duc && (sxon || syon)) sc = ldg(sensp, own_off + (idx_t)kbeg * sz);
+  if (past) ldr(uinp, own_off + (idx_t)kbeg * sz, qn);
+  if (hon) ldr(uinp, h_off + (idx_t)kbeg * sz, uh);
+  if (hpon) ph = ldg(prsp, h_off + (idx_t)kbeg * sz);
+  if (duc && hson) sh = ldg(sensp, h_off + (idx_t)kbeg * sz);
+  {
+    R c[5];
+#pragma unroll
+    for (int v = 0; v < 5; v++) c[v] = own ? q[5][v] : qn[v];
+    put_u(kbeg & 1, c);
+  }
+  put_p(kbeg & 1, qp[2]);
+  if (kbeg < kend) {
+    if (hpon) ph = ldg(prsp, h_off + (idx_t)(kbeg + 1) * sz);
+    put_p((kbeg & 1) ^ 1, qp[3]);
+  }
+  __syncthreads();
+  sensors(kbeg & 1);
+  if (own) {
+    const double sm = duc ? ldg(sensp, own_off + (idx_t)wrap_k(g, kbeg - 1) * sz) : 1.0;
+    const double pm = psens3(qp[0], qp[1], qp[2], sm, cs);
+    ps0 = psens3(qp[1], qp[2], qp[3], sc, cs);
+    const double xk0m = a.xnu0 * fmax(ps0, pm), xk10m = fmax(0.0, a.xnu10 + xk0m / 105.0);
+#pragma unroll
+    for (int v = 0; v < 5; v++) {
+      dlo[v] = (q[5][v] - q[4][v]) * (R)xk0m +
+               (R(D10_1) * (q[5][v] - q[4][v]) + R(D10_2) * (q[6][v] - q[3][v]) + R(D10_3) * (q[7][v] - q[2][v]) +
+                R(D10_4) * (q[8][v] - q[1][v]) + R(D10_5) * (q[9][v] - q[0][v])) *
+                   (R)xk10m;
+    }
+  }
+  // in flight for plane kk = k+1 of the march: the state of the halo and of
+  // points past the end at kk, the queue's kk+4 (and kk+5 from then on), p at
+  // kk+1 and the sensors at kk
+  auto load_ps = [&](int kk) __attribute__((always_inline)) {
+    if (pon) qpn = ldg(prsp, own_off + (idx_t)wrap_k(g, kk + 1) * sz);
+    if (duc && (sxon || syon)) scn = ldg(sensp, own_off + (idx_t)wrap_k(g, kk) * sz);
+    if (kk + 1 <= kend && hpon) ph = ldg(prsp, h_off + (idx_t)(kk + 1) * sz);
+    if (kk <= kend && duc && hson) sh = ldg(sensp, h_off + (idx_t)kk * sz);
+  };
+  if (own) ldr(uinp, own_off + (idx_t)wrap_k(g, kbeg + 5) * sz, qn);
+  if (kbeg < kend) {
+    if (past) ldr(uinp, own_off + (idx_t)(kbeg + 1) * sz, qn);
+    if (hon) ldr(uinp, h_off + (idx_t)(kbeg + 1) * sz, uh);
+  }
+  load_ps(kbeg + 1);
+  __syncthreads();
+
+  for (int k = kbeg; k <= kend; k++) {
+    const idx_t pk = own_off + (idx_t)k * sz;
+    const int b = k & 1;
+    if (own) {
+#pragma unroll
+      for (int v = 0; v < 5; v++) q[10][v] = qn[v];
+    }
+    qp[4] = qpn;
+    sc = scn;
+    if (k < kend) {
+      R c[5];
+#pragma unroll
+      for (int v = 0; v < 5; v++) c[v] = own ? q[6][v] : qn[v];
+      put_u(b ^ 1, c);
+      if (k + 2 <= kend) put_p(b, qp[4]);
+      sensors(b ^ 1);
+      if (own) ldr(uinp, own_off + (idx_t)wrap_k(g, k + 6) * sz, qn);
+      if (k + 2 <= kend) {
+        if (past) ldr(uinp, pk + 2 * sz, qn);
+        if (hon) ldr(uinp, h_off + (idx_t)(k + 2) * sz, uh);
+      }
+      load_ps(k + 2);
+    }
+    if (own) {
+      R K[5];
+      // i faces i-1/2 and i+1/2 (bounded i: rows 1..5 and nx-4..nx take theirs from k_shock_wall)
+      if (WALL && (face_half_n(g.ibnd, g.nx, i - 1) < 5 || face_half_n(g.ibnd, g.nx, i) < 5)) {
+#pragma unroll
+        for (int v = 0; v < 5; v++) K[v] = R(0);
+      } else {
+        const double pm = psx[b][ty][tx], p0 = psx[b][ty][tx + 1], pp = psx[b][ty][tx + 2];
+        const double xk0m = a.xnu0 * fmax(p0, pm), xk10m = fmax(0.0, a.xnu10 + xk0m / 105.0);
+        const double xk0p = a.xnu0 * fmax(pp, p0), xk10p = fmax(0.0, a.xnu10 + xk0p / 105.0);
+#pragma unroll
+        for (int v = 0; v < 5; v++) {
+          const R *x = &su[b][v][ty + 5][tx + 5];
+          K[v] = dface<R>(x - 1, 1, (R)xk0m, (R)xk10m) - dface<R>(x, 1, (R)xk0p, (R)xk10p);
+        }
+      }
+      // j faces (walls: rows 1..5 and ny-4..ny take theirs from k_shock_wall)
+      if (!WALL || (face_half(g, j - 1) >= 5 && face_half(g, j) >= 5)) {
+        const double pm = psy[b][ty][tx], p0 = psy[b][ty + 1][tx], pp = psy[b][ty + 2][tx];
+        const double xk0m = a.xnu0 * fmax(p0, pm), xk10m = fmax(0.0, a.xnu10 + xk0m / 105.0);
+        const double xk0p = a.xnu0 * fmax(pp, p0), xk10p = fmax(0.0, a.xnu10 + xk0p / 105.0);
+#pragma unroll
+        for (int v = 0; v < 5; v++) {
+          const R *y = &su[b][v][ty + 5][tx + 5];
+          K[v] = K[v] + dface<R>(y - SW, SW, (R)xk0m, (R)xk10m) - dface<R>(y, SW, (R)xk0p, (R)xk10p);
+        }
+      }
+      // k face k+1/2 from the register queues
+      {
+        const double pp = psens3(qp[2], qp[3], qp[4], sc, cs);
+        const double xk0p = a.xnu0 * fmax(pp, ps0), xk10p = fmax(0.0, a.xnu10 + xk0p / 105.0);
+        ps0 = pp;
+#pragma unroll
+        for (int v = 0; v < 5; v++) {
+          const R dhi = (q[6][v] - q[5][v]) * (R)xk0p +
+                        (R(D10_1) * (q[6][v] - q[5][v]) + R(D10_2) * (q[7][v] - q[4][v]) +
+                         R(D10_3) * (q[8][v] - q[3][v]) + R(D10_4) * (q[9][v] - q[2][v]) +
+                         R(D10_5) * (q[10][v] - q[1][v])) * (R)xk10p;
+          K[v] = K[v] + dlo[v] - dhi;
+          dlo[v] = dhi;
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < 5; v++) stg_nt(uoutp.v[v], pk, q[5][v] + K[v]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int l = 0; l < 10; l++)
+#pragma unroll
+      for (int v = 0; v < 5; v++) q[l][v] = q[l + 1][v];
+#pragma unroll
+    for (int l = 0; l < 4; l++) qp[l] = qp[l + 1];
+  }
+}
+
 // ARTV: the artificial viscosity.  The LDS "pressure" pencils then hold the
 // spectral radii sr_x (i-pencil) and sr_y (j-pencil), the k queue sr_z.
 // AVS: the artificial viscosity with shock capturing (artvisc_o9_shock,
@@ -297,6 +530,7 @@ __device__ __forceinline__ double edoh_mul(const FilterArgs &a, int d, idx_t p, 
 template <bool ARTV, bool WALL, bool EDOH, bool AVS>
 __global__ __launch_bounds__(FT, 2) void k_filter_shock(const Batch<FilterArgs> *__restrict__ tab, int nb,
                                                         int ntiles) {
+  static_assert(ARTV || EDOH || AVS, "the shock filter alone is k_shock");
   static_assert(!(WALL && ARTV), "walls: not with artvisc_o9");
   static_assert(!(EDOH && (ARTV || AVS)), "the Edoh switch belongs to the shock filter");
   static_assert(!(AVS && ARTV), "one artificial viscosity at a time");
@@ -559,9 +793,7 @@ __global__ __launch_bounds__(FT, 2) void k_filter_shock(const Batch<FilterArgs> 
           const R *x = &sux[v][ty][tx + 5];
           if constexpr (AVS)
             K[v] = (srm * dface<R>(x - 1, 1, (R)xk0m, (R)xk10m) - srp * dface<R>(x, 1, (R)xk0p, (R)xk10p)) * m;
-          else if constexpr (EDOH)
-            K[v] = mul * (dface<R>(x - 1, 1, (R)xk0m, (R)xk10m) - dface<R>(x, 1, (R)xk0p, (R)xk10p));
-          else K[v] = dface<R>(x - 1, 1, (R)xk0m, (R)xk10m) - dface<R>(x, 1, (R)xk0p, (R)xk10p);
+          else K[v] = mul * (dface<R>(x - 1, 1, (R)xk0m, (R)xk10m) - dface<R>(x, 1, (R)xk0p, (R)xk10p));
         }
       }
       // j faces (walls: rows 1..5 and ny-4..ny take theirs from k_shock_wall)
@@ -582,9 +814,7 @@ __global__ __launch_bounds__(FT, 2) void k_filter_shock(const Batch<FilterArgs> 
           if constexpr (AVS)
             K[v] = K[v] +
                    (srm * dface<R>(y - FX, FX, (R)xk0m, (R)xk10m) - srp * dface<R>(y, FX, (R)xk0p, (R)xk10p)) * m;
-          else if constexpr (EDOH)
-            K[v] = K[v] + mul * (dface<R>(y - FX, FX, (R)xk0m, (R)xk10m) - dface<R>(y, FX, (R)xk0p, (R)xk10p));
-          else K[v] = K[v] + dface<R>(y - FX, FX, (R)xk0m, (R)xk10m) - dface<R>(y, FX, (R)xk0p, (R)xk10p);
+          else K[v] = K[v] + mul * (dface<R>(y - FX, FX, (R)xk0m, (R)xk10m) - dface<R>(y, FX, (R)xk0p, (R)xk10p));
         }
       }
       // k faces from the register queues
@@ -612,8 +842,7 @@ __global__ __launch_bounds__(FT, 2) void k_filter_shock(const Batch<FilterArgs> 
                          R(D10_3) * (q[8][v] - q[3][v]) + R(D10_4) * (q[9][v] - q[2][v]) +
                          R(D10_5) * (q[10][v] - q[1][v])) * (R)xk10p;
           if constexpr (AVS) K[v] = K[v] + (srm * dlo - srp * dhi) * m;
-          else if constexpr (EDOH) K[v] = K[v] + mul * (dlo - dhi);
-          else K[v] = K[v] + dlo - dhi;
+          else K[v] = K[v] + mul * (dlo - dhi);
         }
       }
 #pragma unroll
@@ -648,7 +877,7 @@ __constant__ double kShockD[6][5] = {{0.0, 0.0, 0.0, 0.0, 0.0},     {-1.0, 0.0, 
 constexpr int kShockWallThreads = 256;
 
 // Shock filter increment along axis ax (0: i, 1: j) of the rows next to the
-// bounded faces of that axis, added to the output of k_filter_shock<.., WALL>
+// bounded faces of that axis, added to the output of the WALL kernels above
 // (which leaves rows 1..5 and n-4..n of a bounded axis without one): faces
 // 1..4 from a boundary use d2/d4/d6/d8 with amplitude max(0, xnu + xk0), the
 // boundary face a tenth of the sensor term (filter_o10_shock,
@@ -766,8 +995,8 @@ hipError_t launch_filter_shock(const Batch<FilterArgs> *tab, int nb, int nt, Dis
     if (wall) hipLaunchKernelGGL((k_filter_shock<false, true, true, false>), dim3(nt), dim3(FT), 0, s, tab, nb, nt);
     else hipLaunchKernelGGL((k_filter_shock<false, false, true, false>), dim3(nt), dim3(FT), 0, s, tab, nb, nt);
   } else {
-    if (wall) hipLaunchKernelGGL((k_filter_shock<false, true, false, false>), dim3(nt), dim3(FT), 0, s, tab, nb, nt);
-    else hipLaunchKernelGGL((k_filter_shock<false, false, false, false>), dim3(nt), dim3(FT), 0, s, tab, nb, nt);
+    if (wall) hipLaunchKernelGGL((k_shock<true>), dim3(nt), dim3(FT), 0, s, tab, nb, nt);
+    else hipLaunchKernelGGL((k_shock<false>), dim3(nt), dim3(FT), 0, s, tab, nb, nt);
   }
   return hipGetLastError();
 }

@@ -590,11 +590,11 @@ __global__ __launch_bounds__(TX *TY, 2) void k_vdiv(const Batch<VdivArgs> *__res
 // k-gradient comes from a 5-deep queue of the column; the i- and j-fluxes of
 // plane m go through LDS to their differences, which wait two planes for the
 // k-fluxes m-4..m, a ring in LDS (in registers it spilled).  11 waves of at
-// most 168 VGPRs (3 per SIMD), 152 KB of LDS.  Both kernels were bound by
-// memory traffic of which tau and the second metrics read were half; this one
-// by its FP64 arithmetic and LDS accesses at 11 waves per CU.  512x256x128
-// 2.5-D 1118 -> 592 us, 192^3 Cartesian 415 -> 292 us, 256x128x96 c3
-// 294 -> 206 us.
+// most 168 VGPRs (3 per SIMD), 152 KB of LDS.  512x256x128 2.5-D 1118 ->
+// 592 us, 192^3 Cartesian 415 -> 292 us, 256x128x96 c3 294 -> 206 us.  On the
+// first it moves 1.52 GB, 300 us at the rate of a large copy; waves wait for
+// half of their cycles and 25 % more for an issue slot, vector instructions
+// take 17 %.
 constexpr int kFuseThreads = VX * VY + 4 * VY + 4 * VX;
 
 template <int GEO>
