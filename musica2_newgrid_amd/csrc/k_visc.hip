@@ -115,6 +115,10 @@ __device__ __forceinline__ double ducros_of(const double gr[4][3]) {
   return div2 / (div2 + o1 * o1 + o2 * o2 + o3 * o3 + 1.0e-16);
 }
 
+// The gradients and the tensor are written out here, apart from phys_grad and
+// visc_tensor: through them the compiler fuses other multiply-adds, and FP32
+// flux arithmetic carries a changed last bit of K_v on (mixed, 96^3, 50 steps:
+// 1.8e-7 of the state in 1 of 40 runs).
 template <int TX, int TY, int GEO>
 __global__ __launch_bounds__(TX *TY, 2) void k_visc(const Batch<ViscArgs> *__restrict__ tab, int nb, int ntiles) {
   constexpr bool CURV = GEO == kGeoC3;  // 3-D metrics at every point
@@ -259,39 +263,91 @@ __global__ __launch_bounds__(TX *TY, 2) void k_visc(const Batch<ViscArgs> *__res
 
     if (own) {
       const idx_t p = pk;
-      // gradients along the computational directions of u, v, w, T
-      double gd[4][3];
+      // gradients along the computational directions: gd[dir][u,v,w,T]
+      double gd[3][4];
 #pragma unroll
       for (int c = 0; c < 4; c++) {
         const double *fx = &spx[c][ty][tx + 2];
-        gd[c][0] = A5_1 * (fx[1] - fx[-1]) + A5_2 * (fx[2] - fx[-2]);
+        gd[0][c] = A5_1 * (fx[1] - fx[-1]) + A5_2 * (fx[2] - fx[-2]);
         const double *fy = &spy[c][ty + 2][tx];
-        gd[c][1] = A5_1 * (fy[TX] - fy[-TX]) + A5_2 * (fy[2 * TX] - fy[-2 * TX]);
+        gd[1][c] = A5_1 * (fy[TX] - fy[-TX]) + A5_2 * (fy[2 * TX] - fy[-2 * TX]);
       }
-      gd[0][2] = A5_1 * (q[3].u - q[1].u) + A5_2 * (q[4].u - q[0].u);
-      gd[1][2] = A5_1 * (q[3].v - q[1].v) + A5_2 * (q[4].v - q[0].v);
+      gd[2][0] = A5_1 * (q[3].u - q[1].u) + A5_2 * (q[4].u - q[0].u);
+      gd[2][1] = A5_1 * (q[3].v - q[1].v) + A5_2 * (q[4].v - q[0].v);
       gd[2][2] = A5_1 * (q[3].w - q[1].w) + A5_2 * (q[4].w - q[0].w);
-      gd[3][2] = A5_1 * (q[3].T - q[1].T) + A5_2 * (q[4].T - q[0].T);
+      gd[2][3] = A5_1 * (q[3].T - q[1].T) + A5_2 * (q[4].T - q[0].T);
 
-      double gr[4][3], t[NTAU];
-      double ix = 0.0, iy = 0.0, iz = 0.0;
-      if constexpr (!CURV) {
-        iz = ldg(idzv, (idx_t)(k - 1 + G));
-        if constexpr (!C2) {
-          ix = ldg(idxv, (idx_t)(i - 1 + G));
-          iy = ldg(idyv, (idx_t)(j - 1 + G));
+      // physical gradients gr[u,v,w,T][x,y,z]
+      double gr[4][3];
+      if constexpr (C2) {
+        // (f_ksi y_eta - f_eta y_ksi) ijacob, (f_eta x_ksi - f_ksi x_eta) ijacob,
+        // f_z idz (smod_grad_vel_c.f90:186-217, :230-300)
+        const double iz = ldg(idzv, (idx_t)(k - 1 + G));
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          gr[c][0] = (gd[0][c] * mc2[0] + gd[1][c] * mc2[2]) * mc2[4];
+          gr[c][1] = (gd[0][c] * mc2[1] + gd[1][c] * mc2[3]) * mc2[4];
+          gr[c][2] = gd[2][c] * iz;
+        }
+      } else if constexpr (CURV) {
+        const double ij = mvv[9];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          const double dvx = gd[0][c] * mvv[0] + gd[1][c] * mvv[3] + gd[2][c] * mvv[6];
+          const double dvy = gd[0][c] * mvv[1] + gd[1][c] * mvv[4] + gd[2][c] * mvv[7];
+          const double dvz = gd[0][c] * mvv[2] + gd[1][c] * mvv[5] + gd[2][c] * mvv[8];
+          gr[c][0] = dvx * ij;
+          gr[c][1] = dvy * ij;
+          gr[c][2] = dvz * ij;
+        }
+      } else {
+        const double ix = ldg(idxv, (idx_t)(i - 1 + G)), iy = ldg(idyv, (idx_t)(j - 1 + G)), iz = ldg(idzv, (idx_t)(k - 1 + G));
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          gr[c][0] = gd[0][c] * ix;
+          gr[c][1] = gd[1][c] * iy;
+          gr[c][2] = gd[2][c] * iz;
         }
       }
-#pragma unroll
-      for (int c = 0; c < 4; c++) phys_grad<GEO>(gd[c], C2 ? mc2 : mvv, ix, iy, iz, gr[c]);
+
       const double u = q[2].u, v = q[2].v, w = q[2].w, T = q[2].T;
-      visc_tensor(u, v, w, T, gr, a.gas, t);
-#pragma unroll
-      for (int c = 0; c < NTAU; c++) stg(taup[c], p, t[c]);
+      const double mu_l = a.gas.c0 * sqrt(T * T * T) / (T + a.gas.S0) * a.gas.diffscale;
+      const double ck = a.gas.cok_ratio * mu_l;
+
+      double t11 = gr[0][0], t22 = gr[1][1], t33 = gr[2][2];
+      double t12 = 0.5 * (gr[0][1] + gr[1][0]);
+      double t13 = 0.5 * (gr[0][2] + gr[2][0]);
+      double t23 = 0.5 * (gr[1][2] + gr[2][1]);
+      const double tr = (1.0 / 3.0) * (t11 + t22 + t33);
+      const double mu = -2.0 * mu_l;
+      t11 = mu * (t11 - tr);
+      t22 = mu * (t22 - tr);
+      t33 = mu * (t33 - tr);
+      t12 = mu * t12;
+      t13 = mu * t13;
+      t23 = mu * t23;
+
+      stg(taup[0], p, t11);
+      stg(taup[1], p, t12);
+      stg(taup[2], p, t13);
+      stg(taup[3], p, t22);
+      stg(taup[4], p, t23);
+      stg(taup[5], p, t33);
+      stg(taup[6], p, (u * t11 + v * t12 + w * t13) - ck * gr[3][0]);
+      stg(taup[7], p, (u * t12 + v * t22 + w * t23) - ck * gr[3][1]);
+      stg(taup[8], p, (u * t13 + v * t23 + w * t33) - ck * gr[3][2]);
 
       if (a.want_sensor) {
         stg(prsp, p, q[2].p);
-        const double s = a.ducros ? ducros_of(gr) : 1.0;
+        double s = 1.0;
+        if (a.ducros) {
+          const double dv = gr[0][0] + gr[1][1] + gr[2][2];
+          const double div2 = dv * dv;
+          const double o1 = gr[2][1] - gr[1][2];
+          const double o2 = gr[0][2] - gr[2][0];
+          const double o3 = gr[1][0] - gr[0][1];
+          s = div2 / (div2 + o1 * o1 + o2 * o2 + o3 * o3 + 1.0e-16);
+        }
         stg(sensp, p, s);
       }
       if (a.want_sr) {
