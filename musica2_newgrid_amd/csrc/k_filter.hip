@@ -300,9 +300,10 @@ __device__ __forceinline__ double edoh_mul(const FilterArgs &a, int d, idx_t p, 
 // the next and is computed once, as is its pressure sensor.  With three
 // barriers per plane, the plane staged twice (for i and for j) and both k
 // faces of every point: 512x256x128 c3 with walls 876 us, 2.5-D 862 us,
-// 113x75x51 38 us; now 645, 683 and 33 us.  It moves 1.62 GB on the first
-// (320 us at the rate of a large copy): waves wait for 38 % of their cycles
-// and 27 % more for an issue slot, vector instructions take 25 %.
+// 113x75x51 38 us; now 645, 683 and 33 us.  On the first it moves 2.57 GB
+// (1.6 times its words; halo reads), 510 us at the rate of a large copy; waves
+// wait for 38 % of their cycles and 27 % more for an issue slot, vector
+// instructions take 25 %.
 // WALL: blocks with boundary faces on i or j; rows 1..5 and n-4..n of a
 // bounded axis get no increment along it here (k_shock_wall adds it with the
 // reduced faces of the boundary closure).

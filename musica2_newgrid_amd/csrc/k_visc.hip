@@ -648,7 +648,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_vdiv(const Batch<VdivArgs> *__res
 // k-fluxes m-4..m, a ring in LDS (in registers it spilled).  11 waves of at
 // most 168 VGPRs (3 per SIMD), 152 KB of LDS.  512x256x128 2.5-D 1118 ->
 // 592 us, 192^3 Cartesian 415 -> 292 us, 256x128x96 c3 294 -> 206 us.  On the
-// first it moves 1.52 GB, 300 us at the rate of a large copy; waves wait for
+// first it moves 2.24 GB, 445 us at the rate of a large copy; waves wait for
 // half of their cycles and 25 % more for an issue slot, vector instructions
 // take 17 %.
 constexpr int kFuseThreads = VX * VY + 4 * VY + 4 * VX;
